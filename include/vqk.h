@@ -192,6 +192,10 @@ int vqk_grouped_gemm(const vqk_weights *w, const void *x, int32_t x_type,
  * in more panels, less (or none) is VQK_ENOSPACE; it is 16-byte aligned. No
  * host synchronisation, no allocation, no state kept between calls. */
 int vqk_dense_gemm_workspace(const vqk_weights *w, int64_t N, size_t *bytes);
+/* The workspace with which vqk_dense_gemm runs fastest: at least
+ * vqk_dense_gemm_workspace, and for 5..64 rows room for a copy of x in the
+ * matrix cores' operand order (without it x is read in place). */
+int vqk_dense_gemm_scratch(const vqk_weights *w, int64_t N, size_t *bytes);
 int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type,
                    int64_t N, void *y, int32_t y_type, void *workspace,
                    size_t ws_bytes, void *stream);
@@ -361,6 +365,10 @@ int vqk_switch_apply(const vqk_weights *w, const void *x, int32_t x_type,
  * multiplies in x's type). */
 int vqk_linear_apply_workspace(const vqk_weights *w, int64_t N, const vqk_options *o,
                                size_t *bytes);
+/* The workspace with which vqk_linear_apply runs fastest: at least
+ * vqk_linear_apply_workspace, as vqk_dense_gemm_scratch. */
+int vqk_linear_apply_scratch(const vqk_weights *w, int64_t N, const vqk_options *o,
+                             size_t *bytes);
 int vqk_linear_apply(const vqk_weights *w, const void *x, int32_t x_type, int64_t N,
                      void *y, int32_t y_type, void *workspace, size_t ws_bytes,
                      const vqk_options *o, void *stream);

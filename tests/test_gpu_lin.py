@@ -1,0 +1,167 @@
+"""The few-row matrix-core linear (vqk_lin.h) against the float64 oracle: every
+x form, the edges of its row tiles, weight rows longer than one pass, ragged
+last blocks, dead rows, and x that is not finite."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import vq_oracle as vo
+from vq_cases import make_module, skipzero, to_device
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+
+
+def _desc(m, row_table=None, sz=None):
+    from vqlab_amd import _torch as Tt
+    keep = []
+    if sz is not None:
+        codes = torch.from_numpy(np.ascontiguousarray(sz["sz_codes"]).view(np.int32)).cuda()
+        scales = torch.from_numpy(sz["sz_scales"]).cuda()
+        cb = torch.from_numpy(m["codebook"]).cuda()
+        rt = torch.from_numpy(row_table).cuda()
+        return Tt.weights(codes, cb, scales, 64, m["pack_bits"], m["IN"], rt, keep=keep), keep
+    codes, cb, sc = to_device(m)
+    return Tt.weights(codes[0], cb, sc[0], 64, m["pack_bits"], m["IN"], keep=keep), keep
+
+
+def _apply(w, x, scratch=True, fused=64, y_type=torch.float32):
+    """vqk_linear_apply with the fused path up to `fused` rows."""
+    from vqlab_amd import _lib as L, _torch as Tt
+    N = x.shape[0]
+    o = L.options(dense_fused_max_n=fused)
+    ws = ctypes.c_size_t()
+    L.check(L.lib().vqk_linear_apply_scratch(ctypes.byref(w), N, ctypes.byref(o), ctypes.byref(ws)))
+    work = torch.full((max(1, ws.value),), 0xFF, dtype=torch.uint8, device="cuda")
+    y = torch.full((N, w.OUT), float("nan"), dtype=y_type, device="cuda")
+    L.check(L.lib().vqk_linear_apply(ctypes.byref(w), Tt.ptr(x), Tt.act_type(x), N, Tt.ptr(y),
+                                     Tt.act_type(y), Tt.ptr(work) if scratch else None,
+                                     ws.value if scratch else 0, ctypes.byref(o), Tt.stream()))
+    torch.cuda.synchronize()
+    return y.double().cpu().numpy()
+
+
+def _ref(m, x, rounded):
+    """float64 product with the fp16 weight of x rounded to fp16, or (rounded
+    False) of x and the unrounded weight; and the bar of fp32 accumulation:
+    each of the n products and sums of a row rounds once, so n * 2^-24 of
+    sum |w x| bounds the error of any order."""
+    w = vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64).astype(np.float64)
+    if not rounded:
+        w = m["codebook"].astype(np.float64)[m["codes"][0]].reshape(m["OUT"], m["IN"])
+        w = w * np.repeat(m["scales"][0].astype(np.float64), 64, axis=1)
+    xv = x.half() if rounded else x
+    xv = xv.double().cpu().numpy()
+    return xv @ w.T, np.abs(xv) @ np.abs(w).T * (m["IN"] * 2.0 ** -24)
+
+
+# (d, K, packed, OUT, IN): more blocks per row than a GEMV wave holds; ragged
+# last blocks of every width class; OUT off the 16-row tile; a table in LDS,
+# partly in LDS, and not in LDS at all
+SHAPES = [
+    (2, 256, False, 100, 1088), (2, 1024, True, 33, 4224), (4, 256, False, 40, 1344),
+    (4, 4096, True, 130, 8448), (4, 8192, True, 17, 1088), (4, 65536, False, 48, 2048),
+    (8, 4096, True, 65, 1088), (8, 16384, True, 40, 4160), (8, 65536, False, 33, 16640),
+]
+
+
+@pytest.mark.parametrize("d,K,packed,OUT,IN", SHAPES)
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+def test_linear_rows(d, K, packed, OUT, IN, dt):
+    rng = np.random.default_rng(d * 131 + K + IN)
+    m = make_module(rng, 1, OUT, IN, d, K, packed=packed)
+    w, keep = _desc(m)
+    for N in (1, 2, 4, 5, 16, 17, 32, 33, 64):
+        print(f"linear rows d{d} K{K} {IN}->{OUT} {dt} N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda().to(DT[dt])
+        # one row of a shape the block-per-lane GEMV takes is its, which scales
+        # each group's sum (the weight itself not rounded to fp16): 2^-11 more
+        gemv = N == 1 and IN // d % 32 == 0 and IN // d // 32 <= 64
+        ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
+        if gemv:
+            bar = bar + bar / (IN * 2.0 ** -24) * 2.0 ** -11
+        for scratch in (True, False):
+            y = _apply(w, x, scratch)
+            assert (np.abs(y - ref) <= bar).all(), (N, scratch, np.abs(y - ref).max(), bar.min())
+
+
+@pytest.mark.parametrize("d,K,packed", [(2, 1024, True), (4, 4096, True), (8, 16384, True),
+                                        (8, 65536, False)])
+def test_linear_rows_operand_order(d, K, packed):
+    """Shapes whose x is copied into operand order (2^28 products and more),
+    with a ragged last block and an odd OUT, at the edges of the row tiles: the
+    oracle on sampled columns; one row with an infinite value stays alone."""
+    from vqlab_amd import _lib as L
+    rng = np.random.default_rng(d + K)
+    m = make_module(rng, 1, 13001, 4160, d, K, packed=packed)
+    w, keep = _desc(m)
+    cols = np.unique(np.concatenate([rng.choice(m["OUT"], 150, replace=False),
+                                     [0, 15, 16, 12999, 13000]]))
+    sub = dict(m, codes=m["codes"][:, cols], scales=m["scales"][:, cols], OUT=len(cols))
+    for N in (5, 16, 17, 32, 33, 64):
+        print(f"linear operand order d{d} K{K} N{N}", flush=True)
+        o, ws = L.options(dense_fused_max_n=64), ctypes.c_size_t()
+        L.check(L.lib().vqk_linear_apply_scratch(ctypes.byref(w), N, ctypes.byref(o), ctypes.byref(ws)))
+        assert ws.value > 0
+        x = torch.from_numpy(rng.standard_normal((N, m["IN"])).astype(np.float32)).cuda().half()
+        ref, bar = _ref(sub, x, rounded=True)
+        y = _apply(w, x)[:, cols]
+        assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
+        if d != 8:                              # bf16 / fp32 rounded on the way
+            assert np.array_equal(_apply(w, x.float())[:, cols], y)
+        x[1, 7] = float("inf")
+        y = _apply(w, x)
+        assert np.isfinite(y[[0] + list(range(2, N))]).all() and not np.isfinite(y[1]).any()
+
+
+def test_linear_rows_keep_x():
+    """d8 takes bf16 / fp32 x unrounded: values below fp16's smallest and above
+    its largest come through."""
+    rng = np.random.default_rng(5)
+    m = make_module(rng, 1, 48, 2112, 8, 4096)
+    w, keep = _desc(m)
+    for dt in ("bf16", "f32"):
+        print(f"linear keeps x {dt}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((3, m["IN"])).astype(np.float32)).cuda()
+        x[1] *= 2.0 ** -30
+        x[2] *= 2.0 ** 20
+        x = x.to(DT[dt])
+        ref, bar = _ref(m, x, rounded=False)
+        assert (np.abs(_apply(w, x) - ref) <= bar).all()
+
+
+@pytest.mark.parametrize("d,K,IN", [(4, 4096, 1088), (8, 16384, 1088), (2, 1024, 4224)])
+def test_linear_rows_not_finite(d, K, IN):
+    """An infinite or NaN value of one row of x stays in that row, also where
+    the row's end is inside a block (its neighbour's values follow in memory)."""
+    rng = np.random.default_rng(7 + d)
+    m = make_module(rng, 1, 40, IN, d, K)
+    w, keep = _desc(m)
+    for N in (3, 9, 40):
+        print(f"linear not finite d{d} N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda()
+        x[1, 0], x[2, 3] = float("inf"), float("nan")
+        for scratch in (True, False):
+            y = _apply(w, x.half(), scratch)
+            assert np.isfinite(y[[0] + list(range(3, N))]).all()
+            w0 = vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64)[:, 0]
+            assert np.array_equal(y[1][w0 != 0], np.sign(w0[w0 != 0]) * np.inf) and np.isnan(y[2]).all()
+
+
+def test_linear_rows_dead():
+    """Dead skipzero rows are +0, the live ones as in the expanded module."""
+    rng = np.random.default_rng(11)
+    m = make_module(rng, 1, 70, 1088, 4, 4096, dead_frac=0.3)
+    sz, rt = skipzero(m)
+    w, keep = _desc(m, rt, sz)
+    full, keep2 = _desc(m)
+    for N in (3, 20, 40):
+        print(f"linear dead rows N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, m["IN"])).astype(np.float32)).cuda().half()
+        y, ref = _apply(w, x), _apply(full, x)
+        assert np.array_equal(y, ref) and not np.signbit(y[:, rt[0] < 0]).any()

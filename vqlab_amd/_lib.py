@@ -67,6 +67,7 @@ SIGNATURES = {
                                  c_i64, c_p, c_i32, c_p, c_sz, c_p]),
     "vqk_dense_gemm_workspace": (c_i32, [ctypes.POINTER(VQKWeights), c_i64,
                                          ctypes.POINTER(ctypes.c_size_t)]),
+    "vqk_dense_gemm_scratch": (c_i32, [ctypes.POINTER(VQKWeights), c_i64, ctypes.POINTER(c_sz)]),
     "vqk_dense_gemm": (c_i32, [ctypes.POINTER(VQKWeights), c_p, c_i32, c_i64, c_p, c_i32, c_p,
                                ctypes.c_size_t, c_p]),
     "vqk_moe_decode_layer_workspace": (c_i32, [ctypes.POINTER(VQKMoeDesc), c_i64,
@@ -91,6 +92,8 @@ SIGNATURES = {
                                  c_i64, c_p, c_i32, c_p, c_sz, ctypes.POINTER(VQKOptions), c_p]),
     "vqk_linear_apply_workspace": (c_i32, [ctypes.POINTER(VQKWeights), c_i64,
                                            ctypes.POINTER(VQKOptions), ctypes.POINTER(c_sz)]),
+    "vqk_linear_apply_scratch": (c_i32, [ctypes.POINTER(VQKWeights), c_i64,
+                                         ctypes.POINTER(VQKOptions), ctypes.POINTER(c_sz)]),
     "vqk_linear_apply": (c_i32, [ctypes.POINTER(VQKWeights), c_p, c_i32, c_i64, c_p, c_i32, c_p,
                                  c_sz, ctypes.POINTER(VQKOptions), c_p]),
 }

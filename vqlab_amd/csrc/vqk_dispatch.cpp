@@ -5,6 +5,7 @@
 #include <stdlib.h>
 
 #include "vqk_common.h"
+#include "vqk_internal.h"
 
 using namespace vqk;
 
@@ -128,6 +129,16 @@ int vqk_linear_apply_workspace(const vqk_weights *w, int64_t N, const vqk_option
     return vqk_dense_gemm_workspace(w, N, bytes);
 }
 
+int vqk_linear_apply_scratch(const vqk_weights *w, int64_t N, const vqk_options *opt, size_t *bytes) {
+    int rc = vqk_linear_apply_workspace(w, N, opt, bytes);
+    if (rc) return rc;
+    Geom g;
+    if ((rc = make_geom(w, &g))) return rc;
+    const size_t fb = lin_frag_bytes(w, g, N);
+    if (fb > *bytes) *bytes = fb;
+    return VQK_OK;
+}
+
 int vqk_linear_apply(const vqk_weights *w, const void *x, int32_t x_type, int64_t N, void *y,
                      int32_t y_type, void *workspace, size_t ws_bytes, const vqk_options *opt,
                      void *stream) {
@@ -142,7 +153,9 @@ int vqk_linear_apply(const vqk_weights *w, const void *x, int32_t x_type, int64_
         // x's type at every N (vq_dense.py:288-294), so bf16 / fp32 x is
         // taken unrounded here too
         const int32_t xt = g.D == 8 && x_type != VQK_F16 ? (x_type | VQK_X_KEEP) : x_type;
-        return vqk_dense_gemv(w, x, xt, N, y, y_type, stream);
+        if (g.E != 1)
+            return set_error(VQK_EINVAL, "dense GEMV takes one linear (E=1), got E=%lld", (long long)g.E);
+        return launch_gemv(w, x, xt, N, nullptr, N, 1, y, y_type, workspace, ws_bytes, hipStream_t(stream));
     }
     return vqk_dense_gemm(w, x, x_type, N, y, y_type, workspace, ws_bytes, stream);
 }

@@ -625,6 +625,16 @@ int vqk_dense_gemm_workspace(const vqk_weights *w, int64_t N, size_t *bytes) {
     return VQK_OK;
 }
 
+int vqk_dense_gemm_scratch(const vqk_weights *w, int64_t N, size_t *bytes) {
+    int rc = vqk_dense_gemm_workspace(w, N, bytes);
+    if (rc) return rc;
+    Geom g;
+    if ((rc = make_geom(w, &g))) return rc;
+    const size_t fb = N <= kSegDenseMaxN ? lin_frag_bytes(w, g, N) : 0;
+    if (fb > *bytes) *bytes = fb;
+    return VQK_OK;
+}
+
 int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type, int64_t N, void *y,
                    int32_t y_type, void *workspace, size_t ws_bytes, void *stream) {
     Geom g;
@@ -635,6 +645,8 @@ int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type, int64_t 
     if ((rc = check_acts(x, x_type, y, y_type, N))) return rc;
     if (N < 0 || N > INT32_MAX) return set_error(VQK_EINVAL, "N=%lld", (long long)N);
     if (N == 0) return VQK_OK;
+    if (N <= kSegDenseMaxN && lin_ok(w, g, x, x_type, false, N))
+        return launch_lin(w, g, x, x_type, false, N, y, y_type, workspace, ws_bytes, hipStream_t(stream));
     if (N <= kSegDenseMaxN && seg_fits(g, w, x)) {
         SegParams sp;
         fill_seg(w, g, &sp);

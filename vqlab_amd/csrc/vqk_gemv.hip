@@ -45,7 +45,7 @@ size_t gemv_fast_lds(const Geom &g, bool xf) {
 
 int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
                 const uint32_t *eidx, int64_t N, int64_t xkrep, void *y, int32_t y_type,
-                hipStream_t st) {
+                void *ws, size_t ws_bytes, hipStream_t st) {
     Geom g;
     int rc = make_geom(w, &g);
     if (rc) return rc;
@@ -62,6 +62,11 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
                          (long long)N, (long long)T, (long long)xkrep);
     if (N > INT32_MAX) return set_error(VQK_ENOTIMPL, "N=%lld pairs is too many", (long long)N);
     if (N == 0) return VQK_OK;
+    // wide x at d=4: fast instances for the unpacked widths, else the generic kernel
+    const bool fast_x = !xf || g.D == 8 || gemv_fast_d4x_has(g.BITS);
+    const bool fast = g.fast_ok && fast_x && gemv_fast_lds(g, xf) <= size_t(kLdsBytes);
+    if (!eidx && (N > 1 || !fast) && lin_ok(w, g, x, x_type, xf, N))
+        return launch_lin(w, g, x, x_type, xf, N, y, y_type, ws, ws_bytes, st);
     GemvParams p;
     gemv_fill_params(w, g, &p);
     p.eidx = eidx;
@@ -73,9 +78,7 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
     p.y_type = y_type;
     p.y_stride = g.OUT;
     const int64_t chunk = (65535 / xkrep) * xkrep;   // grid.y limit, whole tokens per chunk
-    // wide x at d=4: fast instances for the unpacked widths, else the generic kernel
-    const bool fast_x = !xf || g.D == 8 || gemv_fast_d4x_has(g.BITS);
-    if (g.fast_ok && fast_x && gemv_fast_lds(g, xf) <= size_t(kLdsBytes)) {
+    if (fast) {
         const int rpw = kWave >> p.lpr_log2;
         const int64_t steps_total = N * ((g.OUT + rpw - 1) / rpw);   // wave steps overall
         const int64_t target_waves = 2048;                          // ~8 per CU
@@ -137,14 +140,14 @@ int vqk_dense_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t 
     if (w && w->E != 1)
         return set_error(VQK_EINVAL, "dense GEMV takes one linear (E=1), got E=%lld",
                          (long long)w->E);
-    return launch_gemv(w, x, x_type, N, nullptr, N, 1, y, y_type, hipStream_t(stream));
+    return launch_gemv(w, x, x_type, N, nullptr, N, 1, y, y_type, nullptr, 0, hipStream_t(stream));
 }
 
 int vqk_moe_expert_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
                         const uint32_t *eidx, int64_t N, int64_t xkrep, void *y, int32_t y_type,
                         void *stream) {
     if (!eidx && N > 0) return set_error(VQK_EINVAL, "eidx is required");
-    return launch_gemv(w, x, x_type, T, eidx, N, xkrep, y, y_type, hipStream_t(stream));
+    return launch_gemv(w, x, x_type, T, eidx, N, xkrep, y, y_type, nullptr, 0, hipStream_t(stream));
 }
 
 }  // extern "C"

@@ -15,9 +15,21 @@ int gemv_fill_params(const vqk_weights *w, const Geom &g, GemvParams *p);
 size_t gemv_fast_lds(const Geom &g, bool xf = false);
 
 // Validates and launches the fused GEMV for N = T * xkrep pairs.
+// ws: scratch for one linear's few-row kernel, or NULL (launch_lin).
 int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
                 const uint32_t *eidx, int64_t N, int64_t xkrep, void *y, int32_t y_type,
-                hipStream_t st);
+                void *ws, size_t ws_bytes, hipStream_t st);
+
+// The few-row linear kernel (vqk_lin.h) for N rows of one linear: whether it
+// takes the module and x (xf: x unrounded, VQK_X_KEEP), and its launch.
+bool lin_ok(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N);
+int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N,
+               void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st);
+
+// Workspace that launch_lin makes use of for N rows: the copy of x in the
+// matrix cores' operand order. With less (or none) it reads x in place.
+constexpr int64_t kLinFragRows = 64;
+size_t lin_frag_bytes(const vqk_weights *w, const Geom &g, int64_t N);
 
 // min(items, the current device's CU count): the grid of a kernel that
 // keeps one workgroup per CU (vqk_big.hip).

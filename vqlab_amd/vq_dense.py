@@ -39,7 +39,7 @@ def _decode_matmul(xf, codes_in, codebook, scales, group_size, OUT, IN, pack_bit
     xf = xf.contiguous()
     y = torch.empty((xf.shape[0], int(OUT)), dtype=xf.dtype, device=xf.device)
     ws = ctypes.c_size_t()
-    L.check(L.lib().vqk_dense_gemm_workspace(ctypes.byref(w), xf.shape[0], ctypes.byref(ws)),
+    L.check(L.lib().vqk_dense_gemm_scratch(ctypes.byref(w), xf.shape[0], ctypes.byref(ws)),
             "_decode_matmul")
     work = torch.empty(max(1, ws.value), dtype=torch.uint8, device=xf.device)
     L.check(L.lib().vqk_dense_gemm(ctypes.byref(w), T.ptr(xf), T.act_type(xf), xf.shape[0],
@@ -95,8 +95,8 @@ class VQLinear(torch.nn.Module):
         y = torch.empty((N, OUT), dtype=xf.dtype, device=xf.device)
         o = VS.options()
         ws = ctypes.c_size_t()
-        L.check(L.lib().vqk_linear_apply_workspace(ctypes.byref(w), N, ctypes.byref(o),
-                                                   ctypes.byref(ws)), "VQLinear")
+        L.check(L.lib().vqk_linear_apply_scratch(ctypes.byref(w), N, ctypes.byref(o),
+                                                 ctypes.byref(ws)), "VQLinear")
         work = torch.empty(ws.value, dtype=torch.uint8, device=xf.device) if ws.value else None
         L.check(L.lib().vqk_linear_apply(ctypes.byref(w), T.ptr(xf), T.act_type(xf), N, T.ptr(y),
                                          T.act_type(y), T.ptr(work) if work is not None else None,
