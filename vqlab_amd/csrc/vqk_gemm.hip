@@ -17,6 +17,7 @@
 #include "vqk_gemv.h"
 #include "vqk_gseg.h"
 #include "vqk_internal.h"
+#include "vqk_wide.h"
 
 namespace vqk {
 
@@ -221,6 +222,8 @@ __global__ void __launch_bounds__(64 * WM * WN) k_vq_gemm(const GemmParams p) {
 // the order of pairs follows the atomics; every output row is computed
 // independently, so the results do not depend on it.
 constexpr int kSortThreads = 1024;
+constexpr int kSortUnroll = 8;
+constexpr int kSortLdsPairs = 24 * 1024;       // pair order staged in LDS up to here (96 KB)
 
 __device__ __forceinline__ void block_exclusive_scan(int *a, int n, int *tmp) {
     // a[0..n) in LDS, n <= 4 * kSortThreads; tmp has kSortThreads ints
@@ -231,15 +234,16 @@ __device__ __forceinline__ void block_exclusive_scan(int *a, int n, int *tmp) {
         const int k = tid * per + i;
         if (k < n) local += a[k];
     }
-    tmp[tid] = local;
-    __syncthreads();
-    for (int off = 1; off < kSortThreads; off <<= 1) {
-        const int v = tid >= off ? tmp[tid - off] : 0;
-        __syncthreads();
-        tmp[tid] += v;
-        __syncthreads();
+    int incl = local;                           // inclusive scan of the wave, then of the 16 waves' totals
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int v = __shfl_up(incl, off);
+        if ((tid & (kWave - 1)) >= off) incl += v;
     }
-    int run = tmp[tid] - local;                 // exclusive prefix of this thread's chunk
+    if ((tid & (kWave - 1)) == kWave - 1) tmp[tid / kWave] = incl;
+    __syncthreads();
+    int run = incl - local;                     // exclusive prefix of this thread's chunk
+    for (int w = 0; w < tid / kWave; ++w) run += tmp[w];
+    __syncthreads();
     for (int i = 0; i < per; ++i) {
         const int k = tid * per + i;
         if (k < n) {
@@ -251,9 +255,16 @@ __device__ __forceinline__ void block_exclusive_scan(int *a, int n, int *tmp) {
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(kSortThreads) k_group_sort(const uint32_t *eidx, int N, int E,
-                                                             int BM, int max_tiles, int32_t *order,
-                                                             int32_t *tmeta, int32_t *ntiles) {
+struct SortArgs {
+    const uint32_t *eidx;
+    int N, E, BM, max_tiles;
+    int32_t *order, *tmeta, *ntiles;
+};
+__global__ void __launch_bounds__(kSortThreads) k_group_sort(const SortArgs p) {
+    const uint32_t *eidx = p.eidx;
+    const int N = p.N, E = p.E, max_tiles = p.max_tiles;
+    int BM = p.BM;
+    int32_t *order = p.order, *tmeta = p.tmeta, *ntiles = p.ntiles;
     extern __shared__ int sh[];
     const int NBK = E + 1;
     int *cnt = sh;                 // [NBK] counts, then starts
@@ -265,9 +276,16 @@ __global__ void __launch_bounds__(kSortThreads) k_group_sort(const uint32_t *eid
     for (int b = tid; b < NBK; b += kSortThreads) cnt[b] = 0;
     if (tid < 2) red[tid] = 0;
     __syncthreads();
-    for (int n = tid; n < N; n += kSortThreads) {
-        const uint32_t e = eidx[n];
-        atomicAdd(&cnt[e < uint32_t(E) ? int(e) : E], 1);
+    // ids are read kSortUnroll to a thread at a time: one load's latency (about
+    // a microsecond) for that many instead of for each
+    for (int n0 = tid; n0 < N; n0 += kSortUnroll * kSortThreads) {
+        uint32_t e[kSortUnroll];
+#pragma unroll
+        for (int u = 0; u < kSortUnroll; ++u)
+            e[u] = n0 + u * kSortThreads < N ? eidx[n0 + u * kSortThreads] : 0u;
+#pragma unroll
+        for (int u = 0; u < kSortUnroll; ++u)
+            if (n0 + u * kSortThreads < N) atomicAdd(&cnt[e[u] < uint32_t(E) ? int(e[u]) : E], 1);
     }
     __syncthreads();
     if (BM == kSegTokNarrow) {
@@ -300,12 +318,14 @@ __global__ void __launch_bounds__(kSortThreads) k_group_sort(const uint32_t *eid
     for (int b = tid; b < NBK; b += kSortThreads) {
         const int c = cur[b];
         const int nt = (c + BM - 1) / BM;
+        // wide tiles (multiples of 32 rows) of one bucket share its rows evenly
+        const int per = BM > kSegTok && nt > 0 ? ((c + nt - 1) / nt + 31) / 32 * 32 : BM;
         for (int t = 0; t < nt; ++t) {
             const int ti = tls[b] + t;
             if (ti < max_tiles) {
                 tmeta[3 * ti + 0] = b < E ? b : -1;
-                tmeta[3 * ti + 1] = cnt[b] + t * BM;
-                tmeta[3 * ti + 2] = min(BM, c - t * BM);
+                tmeta[3 * ti + 1] = cnt[b] + t * per;
+                tmeta[3 * ti + 2] = max(0, min(per, c - t * per));
             }
         }
         if (b == NBK - 1) {
@@ -316,10 +336,22 @@ __global__ void __launch_bounds__(kSortThreads) k_group_sort(const uint32_t *eid
     __syncthreads();
     for (int b = tid; b < NBK; b += kSortThreads) cur[b] = cnt[b];
     __syncthreads();
-    for (int n = tid; n < N; n += kSortThreads) {
-        const uint32_t e = eidx[n];
-        const int pos = atomicAdd(&cur[e < uint32_t(E) ? int(e) : E], 1);
-        order[pos] = n;
+    // scattered through LDS where it has the room (one line per store otherwise:
+    // 16384 pairs took 7 us), then written in a row
+    int *dst = N <= kSortLdsPairs ? red + 2 : order;
+    for (int n0 = tid; n0 < N; n0 += kSortUnroll * kSortThreads) {
+        uint32_t e[kSortUnroll];
+#pragma unroll
+        for (int u = 0; u < kSortUnroll; ++u)
+            e[u] = n0 + u * kSortThreads < N ? eidx[n0 + u * kSortThreads] : 0u;
+#pragma unroll
+        for (int u = 0; u < kSortUnroll; ++u)
+            if (n0 + u * kSortThreads < N)
+                dst[atomicAdd(&cur[e[u] < uint32_t(E) ? int(e[u]) : E], 1)] = n0 + u * kSortThreads;
+    }
+    if (dst != order) {
+        __syncthreads();
+        for (int n = tid; n < N; n += kSortThreads) order[n] = dst[n];
     }
 }
 
@@ -537,17 +569,17 @@ int seg_tile_rows(const vqk_weights *w, int64_t N, int64_t E) {
 
 int seg_sort(const uint32_t *eidx, int64_t N, int64_t E, int tok, void *ws, hipStream_t st) {
     if (N == 0) return VQK_OK;
-    if (tok != kSegTok && tok != kSegTokNarrow)
-        return set_error(VQK_EINVAL, "sort tiles of %d rows (16 or %d)", tok, kSegTokNarrow);
+    if (tok != kSegTok && tok != kSegTokNarrow && tok != 64 && tok != 96)
+        return set_error(VQK_EINVAL, "sort tiles of %d rows (16, %d, 64 or 96)", tok, kSegTokNarrow);
     uint8_t *b = static_cast<uint8_t *>(ws);
     const int64_t mt = group_max_tiles(N, E, tok);
     int32_t *order = reinterpret_cast<int32_t *>(b);
     int32_t *tmeta = reinterpret_cast<int32_t *>(b + sort_order_bytes(N));
     int32_t *ntiles = reinterpret_cast<int32_t *>(b + sort_order_bytes(N) + sort_meta_bytes(N, E));
-    const size_t sort_lds = sizeof(int) * (3 * size_t(E + 1) + kSortThreads + 2);
-    hipLaunchKernelGGL(k_group_sort, dim3(1), dim3(kSortThreads), sort_lds, st, eidx, int(N), int(E),
-                       tok, int(mt), order, tmeta, ntiles);
-    return hip_status(hipGetLastError(), "group sort launch");
+    const size_t sort_lds = sizeof(int) * (3 * size_t(E + 1) + kSortThreads + 2 +
+                                           (N <= kSortLdsPairs ? size_t(N) : 0));
+    const SortArgs a{eidx, int(N), int(E), tok, int(mt), order, tmeta, ntiles};
+    return launch_with_lds<k_group_sort>(dim3(1), dim3(kSortThreads), sort_lds, st, a);
 }
 
 int seg_run(const vqk_weights *w, const SegCall &c, const void *sort_ws, hipStream_t st) {
@@ -601,6 +633,104 @@ int seg_run(const vqk_weights *w, const SegCall &c, const void *sort_ws, hipStre
     // the 16-row kernel: dense rows, or sorted tiles of any size (<= 16 rows)
     const dim3 grid{unsigned(nxb), unsigned(tiles), unsigned(ks)};
     return launch_seg(sp, g, kSegTok, grid, st);
+}
+
+static bool wide_module(const vqk_weights *w, const Geom &g) {
+    const bool bits = g.D == 4 ? (g.BITS >= 8 && g.BITS <= 13) : (g.D == 8 && g.BITS >= 8 && g.BITS <= 12);
+    return bits && g.G == 64 && g.NSUB % kBlock == 0 && g.row_words == g.NB * g.BITS && g.rows > 0 &&
+           g.NB * g.BITS <= INT32_MAX && g.IN <= INT32_MAX && g.OUT <= INT32_MAX &&
+           (reinterpret_cast<uintptr_t>(w->codebook) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(w->codes) & 3) == 0;
+}
+
+constexpr int64_t wide_max_x = int64_t(1) << 30;     // elements of x as one buffer of 2 GB
+
+int wide_tile_rows(const vqk_weights *gate, const vqk_weights *up, const vqk_weights *down, int64_t N) {
+    Geom a, b, c;
+    if (make_geom(gate, &a) || make_geom(up, &b) || make_geom(down, &c)) return 0;
+    if (!wide_module(gate, a) || !wide_module(up, b) || !wide_module(down, c) || a.D != b.D ||
+        a.BITS != b.BITS || a.OUT != b.OUT || a.IN != b.IN || a.E != b.E || N * a.IN > wide_max_x ||
+        N * c.IN > wide_max_x)
+        return 0;
+    const int n1 = wide_shape(a.D, a.BITS, true).nt, n2 = wide_shape(c.D, c.BITS, false).nt;
+    return 32 * (n1 < n2 ? n1 : n2);
+}
+
+static void fill_wide(const vqk_weights *w, const Geom &g, WideMod *m) {
+    m->codes = static_cast<const uint32_t *>(w->codes);
+    m->row_words = g.row_words;
+    m->codebook = w->codebook;
+    m->scales = w->scales;
+    m->row_table = w->row_table;
+    m->stored_rows = g.rows;
+    m->K = int32_t(g.K);
+    m->ngrp = int32_t(g.NGRP);
+}
+
+int wide_run(const vqk_weights *w, const vqk_weights *up, const WideCall &c, const void *sort_ws,
+             hipStream_t st) {
+    Geom g;
+    int rc = make_geom(w, &g);
+    if (rc) return rc;
+    if (c.N == 0) return VQK_OK;
+    WideParams p;
+    memset(&p, 0, sizeof p);
+    fill_wide(w, g, &p.m[0]);
+    if (up) {
+        Geom gu;
+        if ((rc = make_geom(up, &gu))) return rc;
+        fill_wide(up, gu, &p.m[1]);
+    }
+    p.E = int32_t(g.E);
+    p.OUT = int32_t(g.OUT);
+    p.IN = int32_t(g.IN);
+    p.NB = int32_t(g.NB);
+    p.x = c.x;
+    const int64_t xrows = c.xkrep ? c.N / c.xkrep : c.N;
+    if (xrows * g.IN > wide_max_x) return set_error(VQK_ENOTIMPL, "x beyond one buffer");
+    p.x_bytes = uint32_t(xrows * g.IN * 2);
+    p.xkrep = int32_t(c.xkrep);
+    p.y = c.y;
+    p.y_type = c.y_type;
+    p.ysorted = up != nullptr;
+    p.N = int32_t(c.N);
+    int64_t tiles;
+    if (sort_ws) {
+        const uint8_t *b = static_cast<const uint8_t *>(sort_ws);
+        p.order = reinterpret_cast<const int32_t *>(b);
+        p.tmeta = reinterpret_cast<const int32_t *>(b + sort_order_bytes(c.N));
+        p.ntiles = reinterpret_cast<const int32_t *>(b + sort_order_bytes(c.N) + sort_meta_bytes(c.N, g.E));
+        tiles = group_max_tiles(c.N, g.E, c.tok);
+    } else {
+        const int nt = wide_shape(g.D, g.BITS, up != nullptr).nt;
+        tiles = (c.N + 32 * nt - 1) / (32 * nt);
+    }
+    if (tiles > 65535) return set_error(VQK_ENOTIMPL, "%lld tiles exceed one launch", (long long)tiles);
+    // A workgroup walks several row blocks -- the table copy and the first
+    // loads' latency are paid once -- while the experts in play still make two
+    // rounds of workgroups: the last round is a smaller part of more (measured
+    // over 64 to 256 experts: within 5 % of the best of 1, 2 and 4).
+    const int64_t nxb = (g.OUT + 255) / 256;
+    const int64_t by_rows = sort_ws ? (c.N + c.tok - 1) / c.tok : tiles, some = g.E < c.N ? g.E : c.N;
+    const int64_t busy = by_rows > some ? by_rows : some;
+    int64_t rb = 1;
+    while (rb < 4 && rb < nxb && busy * ((nxb + 2 * rb - 1) / (2 * rb)) >= 512) rb *= 2;
+    p.rb = int32_t(rb);
+    const dim3 grid(unsigned((nxb + rb - 1) / rb), unsigned(tiles), 1);
+    return g.D == 4 ? launch_wide_d4(p, g.BITS, up != nullptr, grid, st)
+                    : launch_wide_d8(p, g.BITS, up != nullptr, grid, st);
+}
+
+// fp16 copy of activations, 8 per thread
+__global__ void __launch_bounds__(256) k_x_half(const void *x, int x_type, int64_t n8, u32x4 *out) {
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n8) out[i] = load8_act(x, x_type, i * 8);
+}
+
+int launch_x_half(const void *x, int x_type, int64_t n, uint16_t *out, hipStream_t st) {
+    hipLaunchKernelGGL(k_x_half, dim3(unsigned((n / 8 + 255) / 256)), dim3(256), 0, st, x, x_type, n / 8,
+                       reinterpret_cast<u32x4 *>(out));
+    return hip_status(hipGetLastError(), "activation copy launch");
 }
 
 }  // namespace vqk

@@ -40,6 +40,7 @@
 #pragma once
 
 #include <mutex>
+#include <type_traits>
 #include "vqk_common.h"
 
 namespace vqk {
@@ -70,6 +71,15 @@ struct GemvParams {
 };
 
 // ---------------------------------------------------------------- helpers
+// f(integral_constant 0), ..., f(integral_constant N - 1)
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, F, I + 1>(static_cast<F &&>(f));
+    }
+}
+
 template <int D>
 __device__ __forceinline__ float dot_entry(const h2 *cb, uint32_t c, const h2 *x, float acc) {
     if constexpr (D == 2) {

@@ -76,4 +76,25 @@ int seg_sort(const uint32_t *eidx, int64_t N, int64_t E, int tok, void *ws, hipS
 // of expert 0 when sort_ws is NULL).
 int seg_run(const vqk_weights *w, const SegCall &c, const void *sort_ws, hipStream_t st);
 
+// ---- many rows per expert (vqk_wide.h): gate and up at once into fp16 SwiGLU
+// rows in sorted order, then down over those rows.
+struct WideCall {
+    const uint16_t *x;         // fp16 rows, 16-byte aligned
+    int64_t xkrep;             // x row of pair n = n / xkrep; 0: x rows are in sorted order
+    void *y;                   // pair of projections: fp16 [N, OUT] in sorted order; one: y[pair, OUT]
+    int32_t y_type;
+    int64_t N;                 // pairs (sorted) or dense rows (sort_ws == NULL)
+    int32_t tok;               // the sort's tile rows (wide_tile_rows)
+};
+
+// Rows per tile to sort a routing of N pairs into for the projections of a layer,
+// or 0 when the wide kernel does not take them.
+int wide_tile_rows(const vqk_weights *gate, const vqk_weights *up, const vqk_weights *down, int64_t N);
+// `up`: with it, SwiGLU of (w, up). sort_ws: the sorted routing, or NULL for
+// dense rows of one expert.
+int wide_run(const vqk_weights *w, const vqk_weights *up, const WideCall &c, const void *sort_ws,
+             hipStream_t st);
+// fp16 copy of n (a multiple of 8) activations; both 16-byte aligned.
+int launch_x_half(const void *x, int x_type, int64_t n, uint16_t *out, hipStream_t st);
+
 }  // namespace vqk

@@ -286,6 +286,9 @@ __global__ void __launch_bounds__(kLinWaves * 64, lin_waves_per_simd(D, BITS, NT
             pin_words(w);
             asm volatile("" : "+v"(vs));
             if (g + 1 < SPB / GS) look(g + 1, en);
+#ifdef LINSB
+            __builtin_amdgcn_sched_barrier(0);
+#endif
 #pragma unroll
             for (int q = 0; q < GS; ++q) {
                 const int st = g * GS + q;

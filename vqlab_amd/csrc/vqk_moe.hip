@@ -39,6 +39,12 @@ constexpr int kMaxTopK = 64;
 // config-3 layer, T = 16 -> 160 pairs over 512 experts: 698 us sliced GEMV
 // against 745 us grouped; T = 64: 2583 us against 1588 us)
 constexpr int64_t kMoeGroupedMinPairs = 64;
+// pairs per expert from which the grouped projections run as wide tiles
+// (vqk_wide.h; tables of up to 64 KB): level with the 16-row kernel there
+// (256 experts of 2048 x 512, d4 K4096: 33 tokens 151 us against 157) and ahead
+// of it from then on (256 tokens 168 / 198, 2048 tokens 272 / 704; 160 experts
+// of 2560 x 1024, d8 K4096: 128 tokens 204 / 272, 2048 tokens 624 / 2276)
+constexpr int64_t kMoeWideMinPairs = 1;
 
 struct MoeW {            // one projection of the layer, as the kernels see it
     const uint32_t *codes;
@@ -1245,17 +1251,43 @@ __global__ void __launch_bounds__(kWave) k_route_tokens(const MoeParams p) {
     }
 }
 
-// y[t, r] = sum_j w[t, j] * yd[t * k + j, r] + sg[t] * ysh[t, r]
+// y[t, r] = sum_j w[t, j] * yd[t * k + j, r] + sg[t] * ysh[t, r]. Bound by the
+// fp32 rows it reads (134 MB for 2048 tokens x 8 pairs x 2048): four columns to
+// a thread, and eight rows' loads in flight before any is added (in order).
 __global__ void __launch_bounds__(256) k_moe_combine(const MoeParams p, const float *yd,
                                                      const float *ysh) {
     const int t = int(blockIdx.y);
-    const int r = int(blockIdx.x) * 256 + int(threadIdx.x);
+    const int r = (int(blockIdx.x) * 256 + int(threadIdx.x)) * 4;
     if (r >= p.H) return;
-    float acc = 0.f;
-    for (int j = 0; j < p.top_k; ++j)
-        acc += p.wts[t * p.top_k + j] * yd[(int64_t(t) * p.top_k + j) * p.H + r];
-    if (p.shared) acc += p.sg[t] * ysh[int64_t(t) * p.H + r];
-    store_act(p.y, p.y_type, int64_t(t) * p.H + r, acc);
+    const float *w = p.wts + t * p.top_k;
+    const float *src = yd + int64_t(t) * p.top_k * p.H + r;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.H % 4 == 0) {
+        for (int j0 = 0; j0 < p.top_k; j0 += 8) {
+            f32x4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[u] = j0 + u < p.top_k ? *reinterpret_cast<const f32x4 *>(src + int64_t(j0 + u) * p.H)
+                                        : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (j0 + u < p.top_k) {
+                    const float c = w[j0 + u];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] += c * v[u][i];
+                }
+        }
+    } else {
+        for (int j = 0; j < p.top_k; ++j)
+            for (int i = 0; i < 4; ++i)
+                if (r + i < p.H) acc[i] += w[j] * src[int64_t(j) * p.H + i];
+    }
+    for (int i = 0; i < 4; ++i) {
+        if (r + i >= p.H) continue;
+        float a = acc[i];
+        if (p.shared) a += p.sg[t] * ysh[int64_t(t) * p.H + r + i];
+        store_act(p.y, p.y_type, int64_t(t) * p.H + r + i, a);
+    }
 }
 
 // ------------------------------------------------------------ host side
@@ -1682,7 +1714,7 @@ static int launch_moe_big(const vqk_moe_desc *m, const MoePlan &pl, uint8_t *ws,
         if ((rc = launch_gemv_big(b, pl.g2.D, pl.g2.BITS, pl.g2.gpb, dim3(unsigned(big_grid(wg0))), st)))
             return rc;
     }
-    hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 255) / 256), unsigned(T)), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
                        p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
     return hip_status(hipGetLastError(), "combine launch");
 }
@@ -1759,6 +1791,39 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         int r = hip_status(hipEventRecord(ss->e[i], from), "hipEventRecord");
         return r ? r : hip_status(hipStreamWaitEvent(to, ss->e[i], 0), "hipStreamWaitEvent");
     };
+    const int wide = N >= kMoeWideMinPairs * p.E ? wide_tile_rows(m->gate, m->up, m->down, N) : 0;
+    if (wide && (!p.shared || wide_tile_rows(m->sh_gate, m->sh_up, m->sh_down, T))) {
+        // Many rows per expert. x as fp16 rows (where yd goes later) unless it
+        // is; gate and up at once into fp16 SwiGLU rows in sorted order (in g);
+        // down over those. The shared expert is the same over the token rows.
+        const uint16_t *xh = static_cast<const uint16_t *>(p.x);
+        if (p.x_type != VQK_F16) {
+            uint16_t *xc = reinterpret_cast<uint16_t *>(yd);
+            if ((rc = launch_x_half(p.x, p.x_type, T * p.H, xc, st))) return rc;
+            xh = xc;
+        }
+        if ((rc = link(0, st, sb))) return rc;
+        if (p.shared) {
+            const WideCall cs{xh, 1, sgg, VQK_F16, T, 0};
+            if ((rc = wide_run(m->sh_gate, m->sh_up, cs, nullptr, sb))) return rc;
+        }
+        hipLaunchKernelGGL(k_route_tokens, dim3(unsigned(T)), dim3(kWave), 0, st, p);
+        if ((rc = hip_status(hipGetLastError(), "routing launch"))) return rc;
+        if ((rc = seg_sort(reinterpret_cast<const uint32_t *>(p.ids), N, p.E, wide, sort, st))) return rc;
+        const WideCall c{xh, k, g, VQK_F16, N, wide};
+        if ((rc = wide_run(m->gate, m->up, c, sort, st))) return rc;
+        if ((rc = link(1, sb, st))) return rc;                    // down overwrites xh
+        if (p.shared) {
+            const WideCall ds{reinterpret_cast<const uint16_t *>(sgg), 1, ysh, VQK_F32, T, 0};
+            if ((rc = wide_run(m->sh_down, nullptr, ds, nullptr, sb))) return rc;
+        }
+        const WideCall d{reinterpret_cast<const uint16_t *>(g), 0, yd, VQK_F32, N, wide};
+        if ((rc = wide_run(m->down, nullptr, d, sort, st))) return rc;
+        if ((rc = link(3, sb, st))) return rc;
+        hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
+                           p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
+        return hip_status(hipGetLastError(), "combine launch");
+    }
     // the shared expert is one expert over T rows: its gate / up launches
     // alone would fill few CUs, so they split K (fp32 partials that the down
     // launch adds in a fixed order as it stages its input)
@@ -1790,7 +1855,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         if ((rc = seg_run(m->sh_down, ds, nullptr, sb))) return rc;
     }
     if ((rc = link(3, sb, st))) return rc;
-    hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 255) / 256), unsigned(T)), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
                        p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
     return hip_status(hipGetLastError(), "combine launch");
 }
