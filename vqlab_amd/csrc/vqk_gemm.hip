@@ -16,6 +16,7 @@
 // 8*(i/4) + 4*(l/32) + i%4, column l%32.
 #include "vqk_gemv.h"
 #include "vqk_gseg.h"
+#include "vqk_half.h"
 #include "vqk_internal.h"
 #include "vqk_wide.h"
 
@@ -569,8 +570,8 @@ int seg_tile_rows(const vqk_weights *w, int64_t N, int64_t E) {
 
 int seg_sort(const uint32_t *eidx, int64_t N, int64_t E, int tok, void *ws, hipStream_t st) {
     if (N == 0) return VQK_OK;
-    if (tok != kSegTok && tok != kSegTokNarrow && tok != 64 && tok != 96)
-        return set_error(VQK_EINVAL, "sort tiles of %d rows (16, %d, 64 or 96)", tok, kSegTokNarrow);
+    if (tok != kSegTok && tok != kSegTokNarrow && tok != kHalfTile && tok != 64 && tok != 96)
+        return set_error(VQK_EINVAL, "sort tiles of %d rows (16, %d, 32, 64 or 96)", tok, kSegTokNarrow);
     uint8_t *b = static_cast<uint8_t *>(ws);
     const int64_t mt = group_max_tiles(N, E, tok);
     int32_t *order = reinterpret_cast<int32_t *>(b);
@@ -719,6 +720,89 @@ int wide_run(const vqk_weights *w, const vqk_weights *up, const WideCall &c, con
     const dim3 grid(unsigned((nxb + rb - 1) / rb), unsigned(tiles), 1);
     return g.D == 4 ? launch_wide_d4(p, g.BITS, up != nullptr, grid, st)
                     : launch_wide_d8(p, g.BITS, up != nullptr, grid, st);
+}
+
+// Half entries: the one packed width whose d8 table fits LDS by halves and not
+// whole (14 bits), at every row count of the grouped path: 64 tokens of 512
+// experts 848 -> 591 us, 509 tokens 2190 -> 980 us.
+static bool half_module(const vqk_weights *w, const Geom &g) {
+    return g.D == 8 && g.BITS == 14 && g.G == 64 && g.NSUB % kBlock == 0 && g.row_words == g.NB * g.BITS &&
+           g.rows > 0 && g.NB * g.BITS <= INT32_MAX && g.IN <= INT32_MAX && g.OUT <= INT32_MAX - kHalfRows &&
+           (reinterpret_cast<uintptr_t>(w->codebook) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(w->codes) & 3) == 0 && (reinterpret_cast<uintptr_t>(w->scales) & 7) == 0;
+}
+
+bool half_ok(const vqk_weights *gate, const vqk_weights *up, const vqk_weights *down, int64_t N) {
+    Geom a, b, c;
+    if (make_geom(gate, &a) || make_geom(up, &b) || make_geom(down, &c)) return false;
+    return half_module(gate, a) && half_module(up, b) && half_module(down, c) && a.OUT == b.OUT &&
+           a.IN == b.IN && a.E == b.E && N * a.IN <= wide_max_x && N * c.IN <= wide_max_x;
+}
+
+static void fill_half(const vqk_weights *w, const Geom &g, float *const (&y)[2], HalfMod *m) {
+    m->codes = static_cast<const uint32_t *>(w->codes);
+    m->row_words = g.row_words;
+    m->codebook = w->codebook;
+    m->scales = w->scales;
+    m->row_table = w->row_table;
+    m->stored_rows = g.rows;
+    m->K = int32_t(g.K);
+    m->ngrp = int32_t(g.NGRP);
+    m->y[0] = y[0];
+    m->y[1] = y[1];
+}
+
+int half_run(const vqk_weights *w, const vqk_weights *up, const HalfCall &c, const void *sort_ws,
+             hipStream_t st) {
+    static_assert(kHalfTile == kHalfTok, "the sort's tiles are the kernel's");
+    Geom g;
+    int rc = make_geom(w, &g);
+    if (rc) return rc;
+    if (c.N == 0) return VQK_OK;
+    HalfParams p;
+    memset(&p, 0, sizeof p);
+    fill_half(w, g, c.y[0], &p.m[0]);
+    p.nproj = 1;
+    if (up) {
+        Geom gu;
+        if ((rc = make_geom(up, &gu))) return rc;
+        fill_half(up, gu, c.y[1], &p.m[1]);
+        p.nproj = 2;
+    }
+    p.E = int32_t(g.E);
+    p.OUT = int32_t(g.OUT);
+    p.NB = int32_t(g.NB);
+    const int64_t xrows = c.xkrep ? c.N / c.xkrep : c.N;
+    if (xrows * g.IN > wide_max_x) return set_error(VQK_ENOTIMPL, "x beyond one buffer");
+    p.x[0] = c.x;
+    p.x[1] = c.x + xrows * (g.IN / 2);
+    p.x_bytes = uint32_t(xrows * g.IN);
+    p.xkrep = int32_t(c.xkrep);
+    p.ysorted = c.ysorted;
+    p.N = int32_t(c.N);
+    int64_t tiles = (c.N + kHalfTok - 1) / kHalfTok;
+    if (sort_ws) {
+        const uint8_t *b = static_cast<const uint8_t *>(sort_ws);
+        p.order = reinterpret_cast<const int32_t *>(b);
+        p.tmeta = reinterpret_cast<const int32_t *>(b + sort_order_bytes(c.N));
+        p.ntiles = reinterpret_cast<const int32_t *>(b + sort_order_bytes(c.N) + sort_meta_bytes(c.N, g.E));
+        const int64_t some = g.E < c.N ? g.E : c.N;
+        if (tiles < some) tiles = some;
+    }
+    // One workgroup fits a CU (its table): two rounds of them, so that the last
+    // of one launch and the shared expert's beside it even out. A workgroup
+    // takes whole tiles (all row blocks of an expert: one start of its
+    // pipeline) unless that leaves it fewer than four.
+    const int64_t nxb = (g.OUT + kHalfRows - 1) / kHalfRows;
+    const int64_t want = 512 / (2 * p.nproj);
+    int64_t rb = nxb;
+    while (rb > 1 && tiles * ((nxb + rb - 1) / rb) < 4 * want) rb = (rb + 1) / 2;
+    p.rb = int32_t(rb);
+    p.nxg = int32_t((nxb + rb - 1) / rb);
+    const int64_t items = tiles * p.nxg;
+    p.units = int32_t(items < want ? items : want);
+    const int64_t units = int64_t(p.units) * p.nproj;
+    return launch_half(p, g.BITS, dim3(unsigned((units + 7) / 8 * 16)), st);
 }
 
 // fp16 copy of activations, 8 per thread

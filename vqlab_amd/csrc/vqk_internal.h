@@ -94,6 +94,27 @@ int wide_tile_rows(const vqk_weights *gate, const vqk_weights *up, const vqk_wei
 // dense rows of one expert.
 int wide_run(const vqk_weights *w, const vqk_weights *up, const WideCall &c, const void *sort_ws,
              hipStream_t st);
+// ---- d8 tables beyond LDS, halved by entry columns (vqk_half.h): gate and up
+// in one launch, or one projection, into half sums.
+struct HalfCall {
+    const uint16_t *x;         // fp16 half columns [2][rows, IN / 2], 16-byte aligned
+    int64_t xkrep;             // x row of pair n = n / xkrep; 0: x rows are in sorted order
+    float *y[2][2];            // [projection][half] fp32 [N, OUT]
+    bool ysorted;              // y rows in sorted order, not by pair
+    int64_t N;                 // pairs (sorted) or dense rows (sort_ws == NULL)
+};
+// True when the half-entry kernel takes every projection of a layer for N pairs.
+bool half_ok(const vqk_weights *gate, const vqk_weights *up, const vqk_weights *down, int64_t N);
+// `up`: with it, both projections. sort_ws: the routing sorted into tiles of
+// kHalfTile rows, or NULL for dense rows of one expert.
+constexpr int kHalfTile = 32;
+int half_run(const vqk_weights *w, const vqk_weights *up, const HalfCall &c, const void *sort_ws,
+             hipStream_t st);
+// fp16 half columns of n (a multiple of 8) activations, 16-byte aligned, or of
+// SwiGLU rows from half sums.
+int launch_x_split(const void *x, int x_type, int64_t n, uint16_t *out, hipStream_t st);
+int launch_swiglu_split(const float *g0, const float *g1, const float *u0, const float *u1, int64_t n,
+                        uint16_t *out, hipStream_t st);
 // fp16 copy of n (a multiple of 8) activations; both 16-byte aligned.
 int launch_x_half(const void *x, int x_type, int64_t n, uint16_t *out, hipStream_t st);
 

@@ -1254,13 +1254,16 @@ __global__ void __launch_bounds__(kWave) k_route_tokens(const MoeParams p) {
 // y[t, r] = sum_j w[t, j] * yd[t * k + j, r] + sg[t] * ysh[t, r]. Bound by the
 // fp32 rows it reads (134 MB for 2048 tokens x 8 pairs x 2048): four columns to
 // a thread, and eight rows' loads in flight before any is added (in order).
+// yd1, ysh1: the second half sums of each row (vqk_half.h), or NULL.
 __global__ void __launch_bounds__(256) k_moe_combine(const MoeParams p, const float *yd,
-                                                     const float *ysh) {
+                                                     const float *ysh, const float *yd1,
+                                                     const float *ysh1) {
     const int t = int(blockIdx.y);
     const int r = (int(blockIdx.x) * 256 + int(threadIdx.x)) * 4;
     if (r >= p.H) return;
     const float *w = p.wts + t * p.top_k;
     const float *src = yd + int64_t(t) * p.top_k * p.H + r;
+    const float *src1 = yd1 + (yd1 ? int64_t(t) * p.top_k * p.H + r : 0);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (p.H % 4 == 0) {
         for (int j0 = 0; j0 < p.top_k; j0 += 8) {
@@ -1269,6 +1272,15 @@ __global__ void __launch_bounds__(256) k_moe_combine(const MoeParams p, const fl
             for (int u = 0; u < 8; ++u)
                 v[u] = j0 + u < p.top_k ? *reinterpret_cast<const f32x4 *>(src + int64_t(j0 + u) * p.H)
                                         : f32x4{0.f, 0.f, 0.f, 0.f};
+            if (yd1) {
+                f32x4 v1[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    v1[u] = j0 + u < p.top_k ? *reinterpret_cast<const f32x4 *>(src1 + int64_t(j0 + u) * p.H)
+                                             : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] += v1[u];
+            }
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (j0 + u < p.top_k) {
@@ -1280,12 +1292,16 @@ __global__ void __launch_bounds__(256) k_moe_combine(const MoeParams p, const fl
     } else {
         for (int j = 0; j < p.top_k; ++j)
             for (int i = 0; i < 4; ++i)
-                if (r + i < p.H) acc[i] += w[j] * src[int64_t(j) * p.H + i];
+                if (r + i < p.H)
+                    acc[i] += w[j] * (src[int64_t(j) * p.H + i] + (yd1 ? src1[int64_t(j) * p.H + i] : 0.f));
     }
     for (int i = 0; i < 4; ++i) {
         if (r + i >= p.H) continue;
         float a = acc[i];
-        if (p.shared) a += p.sg[t] * ysh[int64_t(t) * p.H + r + i];
+        if (p.shared) {
+            const int64_t n = int64_t(t) * p.H + r + i;
+            a += p.sg[t] * (ysh[n] + (ysh1 ? ysh1[n] : 0.f));
+        }
         store_act(p.y, p.y_type, int64_t(t) * p.H + r + i, a);
     }
 }
@@ -1301,6 +1317,9 @@ struct MoeLayout {
     size_t g, u, sgg, sgu, yd, ysh;      // composed paths (sliced-codebook GEMV, grouped GEMM)
     size_t sort;                         // grouped path: pair order and tile records
     size_t gs, us;                       // fused path, split K1: fp32 gate / up rows
+    // grouped path over half entries (vqk_half.h), after `total`: a workspace of
+    // `total` bytes alone runs the call without it
+    size_t hs, hsh, y1, ysh1, full;
 };
 
 // Paths of the layer: the two fused decode kernels, the sliced-codebook GEMV
@@ -1309,7 +1328,7 @@ struct MoeLayout {
 enum MoePath { kMoeFused = 0, kMoeBig = 1, kMoeGrouped = 2 };
 
 static MoeLayout moe_layout(int64_t T, int k, int P, int64_t I, int64_t H, int path, int64_t E,
-                            bool split) {
+                            bool split, bool half) {
     MoeLayout L;
     L.ids = kHdrBytes;
     L.wts = align_up(L.ids + sizeof(int32_t) * T * k);
@@ -1337,6 +1356,17 @@ static MoeLayout moe_layout(int64_t T, int k, int P, int64_t I, int64_t H, int p
         L.sort = L.total;
         L.total = align_up(L.sort + seg_sort_bytes(T * k, E));
     }
+    L.hs = L.hsh = L.y1 = L.ysh1 = 0;
+    L.full = L.total;
+    if (half) {
+        // second half sums: gate and up rows, later down's in their place
+        const size_t n = size_t(T) * k, gu = 8 * n * I, dn = 4 * n * H;
+        L.hs = L.total;
+        L.hsh = align_up(L.hs + 2 * n * I);
+        L.y1 = align_up(L.hsh + 2 * size_t(T) * I);
+        L.ysh1 = align_up(L.y1 + (gu > dn ? gu : dn));
+        L.full = align_up(L.ysh1 + 4 * size_t(T) * H);
+    }
     return L;
 }
 
@@ -1362,6 +1392,7 @@ struct MoePlan {
     size_t smem1, smem2;
     dim3 grid1, grid2;
     int path;                 // MoePath
+    bool half;                // grouped path over half entries, given its workspace
     bool split;               // fused path, tables beyond LDS: one projection per K1 workgroup
     bool wide1, wide2;        // the larger LDS parts of a partly staged table fit
     bool l1;                  // fused path as one launch (k_moe_layer1)
@@ -1531,7 +1562,9 @@ static int moe_plan(const vqk_moe_desc *m, int64_t T, MoePlan *pl) {
     if (pl->path == kMoeFused && (pl->smem1 > 160 * 1024 || pl->smem2 > 160 * 1024))
         return set_error(VQK_ENOTIMPL, "fused layer: LDS need %zu / %zu B exceeds 160 KB",
                          pl->smem1, pl->smem2);
-    pl->lay = moe_layout(T, k, P, gg.OUT, gg.IN, pl->path, E, pl->split);
+    pl->half = pl->path == kMoeGrouped && half_ok(m->gate, m->up, m->down, N) &&
+               (!shared || half_ok(m->sh_gate, m->sh_up, m->sh_down, T));
+    pl->lay = moe_layout(T, k, P, gg.OUT, gg.IN, pl->path, E, pl->split, pl->half);
     // One launch: batch 1, gate/up and down workgroups resident together, two
     // per CU (LDS and 128 VGPRs each), tables in LDS (a shared expert's down
     // table beside the routed one), one format, the stamps and words within
@@ -1715,7 +1748,7 @@ static int launch_moe_big(const vqk_moe_desc *m, const MoePlan &pl, uint8_t *ws,
             return rc;
     }
     hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
-                       p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
+                       p, static_cast<const float *>(yd), static_cast<const float *>(ysh), static_cast<const float *>(nullptr), static_cast<const float *>(nullptr));
     return hip_status(hipGetLastError(), "combine launch");
 }
 
@@ -1821,7 +1854,41 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         if ((rc = wide_run(m->down, nullptr, d, sort, st))) return rc;
         if ((rc = link(3, sb, st))) return rc;
         hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
-                           p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
+                           p, static_cast<const float *>(yd), static_cast<const float *>(ysh), static_cast<const float *>(nullptr), static_cast<const float *>(nullptr));
+        return hip_status(hipGetLastError(), "combine launch");
+    }
+    if (pl.half) {
+        // d8 tables beyond LDS, each workgroup with half of every entry: x and
+        // the SwiGLU rows as half columns, every projection's two half sums
+        // added by what reads them. The shared expert is the same over the
+        // token rows.
+        const float *none = nullptr;
+        uint16_t *xh = reinterpret_cast<uint16_t *>(yd);          // until down overwrites it
+        uint16_t *hs = reinterpret_cast<uint16_t *>(ws + pl.lay.hs), *hsh = reinterpret_cast<uint16_t *>(ws + pl.lay.hsh);
+        float *y1 = reinterpret_cast<float *>(ws + pl.lay.y1), *ysh1 = reinterpret_cast<float *>(ws + pl.lay.ysh1);
+        if ((rc = launch_x_split(p.x, p.x_type, T * p.H, xh, st))) return rc;
+        if ((rc = link(0, st, sb))) return rc;
+        if (p.shared) {
+            float *sg1 = sgg + T * p.I, *su1 = sgu + T * p.I;
+            const HalfCall cs{xh, 1, {{sgg, sg1}, {sgu, su1}}, true, T};
+            if ((rc = half_run(m->sh_gate, m->sh_up, cs, nullptr, sb))) return rc;
+            if ((rc = launch_swiglu_split(sgg, sg1, sgu, su1, T * p.I, hsh, sb))) return rc;
+            const HalfCall ds{hsh, 0, {{ysh, ysh1}, {}}, true, T};
+            if ((rc = half_run(m->sh_down, nullptr, ds, nullptr, sb))) return rc;
+        }
+        hipLaunchKernelGGL(k_route_tokens, dim3(unsigned(T)), dim3(kWave), 0, st, p);
+        if ((rc = hip_status(hipGetLastError(), "routing launch"))) return rc;
+        if ((rc = seg_sort(reinterpret_cast<const uint32_t *>(p.ids), N, p.E, kHalfTile, sort, st))) return rc;
+        float *g1 = y1, *u1 = y1 + N * p.I;
+        const HalfCall c{xh, k, {{g, g1}, {u, u1}}, true, N};
+        if ((rc = half_run(m->gate, m->up, c, sort, st))) return rc;
+        if ((rc = launch_swiglu_split(g, g1, u, u1, N * p.I, hs, st))) return rc;
+        if ((rc = link(1, sb, st))) return rc;                    // down overwrites xh
+        const HalfCall d{hs, 0, {{yd, y1}, {}}, false, N};
+        if ((rc = half_run(m->down, nullptr, d, sort, st))) return rc;
+        hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
+                           p, static_cast<const float *>(yd), static_cast<const float *>(ysh),
+                           static_cast<const float *>(y1), p.shared ? static_cast<const float *>(ysh1) : none);
         return hip_status(hipGetLastError(), "combine launch");
     }
     // the shared expert is one expert over T rows: its gate / up launches
@@ -1856,7 +1923,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
     }
     if ((rc = link(3, sb, st))) return rc;
     hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
-                       p, static_cast<const float *>(yd), static_cast<const float *>(ysh));
+                       p, static_cast<const float *>(yd), static_cast<const float *>(ysh), static_cast<const float *>(nullptr), static_cast<const float *>(nullptr));
     return hip_status(hipGetLastError(), "combine launch");
 }
 
@@ -1973,7 +2040,7 @@ int vqk_moe_decode_layer_workspace(const vqk_moe_desc *m, int64_t T, size_t *byt
     MoePlan pl;
     int rc = moe_plan(m, T, &pl);
     if (rc) return rc;
-    *bytes = pl.lay.total;
+    *bytes = pl.lay.full;
     return VQK_OK;
 }
 
@@ -2009,6 +2076,7 @@ int vqk_moe_decode_layer(const vqk_moe_desc *m, const void *x, int32_t x_type, i
     if (pl.path == kMoeGrouped) {
         if ((reinterpret_cast<uintptr_t>(x) & 15) != 0)
             return set_error(VQK_EINVAL, "batched layer: x must be 16-byte aligned");
+        pl.half = pl.half && ws_bytes >= pl.lay.full;
         return launch_moe_grouped(m, pl, ws, st);
     }
     if (pl.path == kMoeBig) return launch_moe_big(m, pl, ws, st);
