@@ -68,6 +68,26 @@ def test_vq_embedding_ids_outside_table_give_zero_rows():
     assert not g[[1, 2, 4]].any()
 
 
+@pytest.mark.parametrize("D,K,IN,G", [(4, 4096, 96, 24), (8, 32, 72, 8), (4, 2, 8, 8), (8, 65536, 264, 88)])
+@pytest.mark.parametrize("out_dtype", ["float16", "bfloat16", "float32"])
+def test_vq_embedding_block_rows(D, K, IN, G, out_dtype):
+    """Block-packed rows whose chunks lie in one scale group: groups that are
+    no power of two, rows of one chunk, widths of 1 to 16 bits, a partly filled
+    last workgroup, ids outside the table among the others."""
+    from vqlab_amd.vq_dense import VQEmbedding
+    print(f"VQEmbedding blocks D={D} K={K} IN={IN} G={G} out={out_dtype}", flush=True)
+    od = getattr(torch, out_dtype)
+    rng = np.random.default_rng(D + K + IN)
+    m = make_module(rng, 1, 61, IN, D, K, G=G, packed=True)
+    codes, cb, sc = to_device(m)
+    emb = VQEmbedding(codes[0], cb, sc[0], group_size=G, pack_bits=m["pack_bits"], in_features=IN, out_dtype=od)
+    ids = rng.integers(-2, 63, 77)
+    ok = (ids >= 0) & (ids < 61)
+    got = _bits(emb(torch.from_numpy(ids).cuda()))
+    ref = vo.embed_rows(ids[ok], m["codes"][0], m["codebook"], m["scales"][0], G)
+    assert np.array_equal(got[ok], _expect(ref, od)) and not got[~ok].any()
+
+
 def test_vq_embedding_empty_ids_and_sharded_codebook():
     from vqlab_amd.vq_dense import VQEmbedding
     rng = np.random.default_rng(6)

@@ -16,6 +16,8 @@
 //   byte stream   uint8 [row_bytes]: code j at bits [j*bits, (j+1)*bits) of the
 //                 row, LSB first -- the PLE shard format, read through a
 //                 3-byte window at byte (j*bits)/8 (vq_switch.py:5449-5470)
+#include <type_traits>
+
 #include "vqk_common.h"
 #include "vqk_gemv.h"
 
@@ -131,6 +133,57 @@ __global__ void __launch_bounds__(256) k_embed_gather(const EmbedArgs a) {
     }
 }
 
+// The same for block-packed codes of d = 4 or 8 and scale groups of whole
+// chunks: a lane's eight outputs are one or two entries under one scale. The
+// general kernel divides 64-bit indexes by d and the group for every output
+// and reads code and scale again for each; 2048 rows of 4096, d4 K4096 (20 MB):
+// the kernel 25 us -> 9.3, the call 22.5 -> 14.7 (MI355X), which is its host path.
+template <int D>
+__global__ void __launch_bounds__(256) k_embed_blocks(const EmbedArgs a) {
+    constexpr int NC = 8 / D;
+    const uint32_t it = blockIdx.x * 256u + threadIdx.x, lpr = uint32_t(a.lanes_per_row);
+    const uint32_t i = it / lpr, j0 = (it - i * lpr) * 8u;
+    if (int64_t(i) >= a.n) return;
+    const int64_t id = a.id64 ? static_cast<const int64_t *>(a.ids)[i]
+                              : int64_t(static_cast<const int32_t *>(a.ids)[i]);
+    uint16_t h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (id >= 0 && id < a.rows) {               // ids outside the table give rows of +0
+        const float s = h_to_f32(a.scales[id * a.ngrp + j0 / uint32_t(a.G)]);
+        typedef typename std::conditional<D == 4, u32x2, u32x4>::type Entry;
+        Entry e[NC];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const uint32_t code = embed_code(a, id, int64_t(j0 / D + q));
+            e[q] = reinterpret_cast<const Entry *>(a.codebook)[min(code, uint32_t(a.K - 1))];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const uint32_t w = e[t / D][(t % D) / 2];
+            h[t] = f32_to_h(h_to_f32(uint16_t(t & 1 ? w >> 16 : w & 0xffffu)) * s);
+        }
+    }
+    const int64_t o = int64_t(i) * a.IN + j0;
+    if (a.out_type == VQK_F32) {
+        u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<float *>(a.out) + o);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            u32x4 v;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) v[t] = __float_as_uint(h_to_f32(h[4 * q + t]));
+            dst[q] = v;
+        }
+        return;
+    }
+    if (a.out_type == VQK_BF16) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) h[t] = h_to_bf16(h[t]);
+    }
+    u32x4 v;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = uint32_t(h[2 * t]) | (uint32_t(h[2 * t + 1]) << 16);
+    *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(a.out) + o) = v;
+}
+
 // Validates an embedding table descriptor (E == 1, OUT = table rows) and
 // fills the layout fields of `a`.
 static int embed_args(const vqk_weights *w, EmbedArgs *a) {
@@ -227,6 +280,14 @@ int vqk_embed_gather(const vqk_weights *w, const void *ids, int32_t id_type, int
     a.vec_ok = (a.IN % 8 == 0) && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     const int64_t total = n * a.lanes_per_row;
     const int64_t blocks = (total + 255) / 256;
+    // 32-bit indexes, 16-byte entries of d = 8 and 8-byte ones of d = 4: ahead of
+    // the general kernel wherever it applies (25 against 9.3 us, above)
+    if (a.layout == kEmbBlocks && (a.D == 4 || a.D == 8) && a.G % 8 == 0 && a.vec_ok &&
+        (reinterpret_cast<uintptr_t>(w->codebook) & 15) == 0 && total <= INT32_MAX && a.IN <= INT32_MAX) {
+        if (a.D == 4) hipLaunchKernelGGL(k_embed_blocks<4>, dim3(unsigned(blocks)), dim3(256), 0, hipStream_t(stream), a);
+        else hipLaunchKernelGGL(k_embed_blocks<8>, dim3(unsigned(blocks)), dim3(256), 0, hipStream_t(stream), a);
+        return hip_status(hipGetLastError(), "embedding gather launch");
+    }
     const unsigned grid = unsigned(blocks < 65536 ? blocks : 65536);
     hipLaunchKernelGGL(k_embed_gather, dim3(grid), dim3(256), 0, hipStream_t(stream), a);
     return hip_status(hipGetLastError(), "embedding gather launch");
