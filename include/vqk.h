@@ -243,6 +243,9 @@ typedef struct vqk_moe_desc {
     int32_t            norm_topk;
 } vqk_moe_desc;
 
+/* The workspace with which the call runs fastest. For d8 tables of 14-bit
+ * codes in a grouped call it includes the second half sums of each row; a
+ * workspace without them still runs the call, on the 16-row kernels. */
 int vqk_moe_decode_layer_workspace(const vqk_moe_desc *m, int64_t T,
                                    size_t *bytes);
 int vqk_moe_decode_layer(const vqk_moe_desc *m, const void *x, int32_t x_type,
@@ -267,8 +270,8 @@ int vqk_moe_layer_reset(void *workspace, void *stream);
  * vqk_moe_decode_layer, without the workspace: the layer's scratch is a
  * library-owned device array of VQK_NOALLOC_SCRATCH_BYTES per GPU, taken when
  * the library is loaded on that GPU and held until the process ends. A call
- * whose workspace (vqk_moe_decode_layer_workspace) exceeds it returns
- * VQK_ENOSPACE before any launch (config 4 at T = 64 needs about 19 MB).
+ * whose smallest workspace exceeds it returns VQK_ENOSPACE before any launch
+ * (config 4 at T = 64 needs about 19 MB).
  * Every call on one GPU shares that GPU's array: calls that overlap on one
  * GPU (two streams, two threads) race and must be serialised by the caller.
  * The array starts zeroed (static device storage), which its header needs;
