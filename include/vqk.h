@@ -147,7 +147,9 @@ int vqk_dequant_experts(const vqk_weights *w, const uint32_t *eidx,
 
 /* ---- a10: dense fused GEMV, _dense_fused (vq_switch.py:3339-3434) ----------
  * y[N, OUT] = x[N, IN] . W^T for E == 1, fp32 accumulation; x and y types in
- * {VQK_F16, VQK_BF16, VQK_F32}. */
+ * {VQK_F16, VQK_BF16, VQK_F32}. At every N each scale multiplies the fp32 sum
+ * of its group's products of entry and x (the weight entry * scale is not
+ * rounded to fp16). */
 int vqk_dense_gemv(const vqk_weights *w, const void *x, int32_t x_type,
                    int64_t N, void *y, int32_t y_type, void *stream);
 
@@ -177,9 +179,9 @@ int vqk_grouped_gemm(const vqk_weights *w, const void *x, int32_t x_type,
                      void *stream);
 
 /* ---- a11: dense large-N path, _decode_matmul (vq_dense.py:262-312) ---------
- * y[N, OUT] = x[N, IN] . W^T for E == 1. Up to 64 rows: W is decoded straight
- * into matrix-core operands (no workspace, x rounded to fp16 as the fused
- * kernels take it). Above (and for shapes that path refuses): the reference's
+ * y[N, OUT] = x[N, IN] . W^T for E == 1. Up to 64 rows: W = fp16(cb * s) is
+ * decoded straight into matrix-core operands (no workspace, x rounded to fp16
+ * as the fused kernels take it). Above (and for shapes that path refuses): the reference's
  * decode-then-matmul, `xf @ w.T.astype(xf.dtype)` -- W is dequantised into the
  * workspace panel by panel in x's arithmetic type and multiplied by libvqk's
  * matrix-core GEMM with fp32 accumulation: fp16 x against the bit-exact fp16

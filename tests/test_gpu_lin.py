@@ -46,15 +46,21 @@ def _apply(w, x, scratch=True, fused=64, y_type=torch.float32):
     return y.double().cpu().numpy()
 
 
-def _ref(m, x, rounded):
-    """float64 product with the fp16 weight of x rounded to fp16, or (rounded
-    False) of x and the unrounded weight; and the bar of fp32 accumulation:
-    each of the n products and sums of a row rounds once, so n * 2^-24 of
-    sum |w x| bounds the error of any order."""
-    w = vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64).astype(np.float64)
-    if not rounded:
-        w = m["codebook"].astype(np.float64)[m["codes"][0]].reshape(m["OUT"], m["IN"])
-        w = w * np.repeat(m["scales"][0].astype(np.float64), 64, axis=1)
+def _weight(m, decoded):
+    """float64 [OUT, IN]: the fp16 weight that the dequant writes, or (decoded
+    False) the unrounded product of entry and scale."""
+    if decoded:
+        return vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64).astype(np.float64)
+    w = m["codebook"].astype(np.float64)[m["codes"][0]].reshape(m["OUT"], m["IN"])
+    return w * np.repeat(m["scales"][0].astype(np.float64), 64, axis=1)
+
+
+def _ref(m, x, rounded, decoded=False):
+    """float64 product of x, or x rounded to fp16, with the module's weight;
+    and the bar of fp32 accumulation: each of the n products and sums of a row,
+    and the scaling of its groups' sums, rounds once, so n * 2^-24 of sum |w x|
+    bounds the error of any order (n / 64 scalings, well under the n sums)."""
+    w = _weight(m, decoded)
     xv = x.half() if rounded else x
     xv = xv.double().cpu().numpy()
     return xv @ w.T, np.abs(xv) @ np.abs(w).T * (m["IN"] * 2.0 ** -24)
@@ -79,12 +85,7 @@ def test_linear_rows(d, K, packed, OUT, IN, dt):
     for N in (1, 2, 4, 5, 16, 17, 32, 33, 64):
         print(f"linear rows d{d} K{K} {IN}->{OUT} {dt} N{N}", flush=True)
         x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda().to(DT[dt])
-        # one row of a shape the block-per-lane GEMV takes is its, which scales
-        # each group's sum (the weight itself not rounded to fp16): 2^-11 more
-        gemv = N == 1 and IN // d % 32 == 0 and IN // d // 32 <= 64
         ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
-        if gemv:
-            bar = bar + bar / (IN * 2.0 ** -24) * 2.0 ** -11
         for scratch in (True, False):
             y = _apply(w, x, scratch)
             assert (np.abs(y - ref) <= bar).all(), (N, scratch, np.abs(y - ref).max(), bar.min())
@@ -117,6 +118,30 @@ def test_linear_rows_operand_order(d, K, packed):
         x[1, 7] = float("inf")
         y = _apply(w, x)
         assert np.isfinite(y[[0] + list(range(2, N))]).all() and not np.isfinite(y[1]).any()
+
+
+@pytest.mark.parametrize("d,K,packed", [(2, 1024, True), (4, 4096, True), (8, 4096, True),
+                                        (8, 65536, False)])
+def test_linear_rows_scale_in_fp32(d, K, packed):
+    """The scale multiplies a group's fp32 sum, not the fp16 entry: products of
+    entry and scale above fp16's range (rows 0, 3, ...) and among its subnormals
+    (rows 1, 4, ...) come out as exactly as the others, whatever the row count;
+    IN leaves the last superstep one block and half a block."""
+    rng = np.random.default_rng(d + K)
+    m = make_module(rng, 1, 50, 64 * 33, d, K, packed=packed, cb_std=2.0)
+    m["scales"][0, 0::3] *= np.float16(40000)
+    m["scales"][0, 1::3] *= np.float16(2.0 ** -12)
+    m["codebook"][: K // 2] *= np.float16(2.0 ** -10)
+    w, keep = _desc(m)
+    prod = np.abs(_weight(m, False))
+    assert prod.max() > 65504 and (prod[1::3] < 2.0 ** -14).mean() > 0.5
+    for dt in DT:
+        for N in (2, 7, 16, 20, 32):
+            print(f"linear scale d{d} K{K} {dt} N{N}", flush=True)
+            x = torch.from_numpy(rng.standard_normal((N, m["IN"])).astype(np.float32)).cuda().to(DT[dt])
+            ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
+            y = _apply(w, x)
+            assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
 
 
 def test_linear_rows_keep_x():

@@ -860,7 +860,7 @@ int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type, int64_t 
     if (N < 0 || N > INT32_MAX) return set_error(VQK_EINVAL, "N=%lld", (long long)N);
     if (N == 0) return VQK_OK;
     if (N <= kSegDenseMaxN && lin_ok(w, g, x, x_type, false, N))
-        return launch_lin(w, g, x, x_type, false, N, y, y_type, workspace, ws_bytes, hipStream_t(stream));
+        return launch_lin(w, g, x, x_type, false, true, N, y, y_type, workspace, ws_bytes, hipStream_t(stream));
     if (N <= kSegDenseMaxN && seg_fits(g, w, x)) {
         SegParams sp;
         fill_seg(w, g, &sp);

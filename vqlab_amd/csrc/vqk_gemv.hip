@@ -66,7 +66,7 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
     const bool fast_x = !xf || g.D == 8 || gemv_fast_d4x_has(g.BITS);
     const bool fast = g.fast_ok && fast_x && gemv_fast_lds(g, xf) <= size_t(kLdsBytes);
     if (!eidx && (N > 1 || !fast) && lin_ok(w, g, x, x_type, xf, N))
-        return launch_lin(w, g, x, x_type, xf, N, y, y_type, ws, ws_bytes, st);
+        return launch_lin(w, g, x, x_type, xf, false, N, y, y_type, ws, ws_bytes, st);
     GemvParams p;
     gemv_fill_params(w, g, &p);
     p.eidx = eidx;

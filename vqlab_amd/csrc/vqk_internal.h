@@ -23,8 +23,8 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
 // The few-row linear kernel (vqk_lin.h) for N rows of one linear: whether it
 // takes the module and x (xf: x unrounded, VQK_X_KEEP), and its launch.
 bool lin_ok(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N);
-int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N,
-               void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st);
+int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, bool deq,
+               int64_t N, void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st);
 
 // Workspace that launch_lin makes use of for N rows: the copy of x in the
 // matrix cores' operand order. With less (or none) it reads x in place.

@@ -37,8 +37,8 @@ size_t lin_frag_bytes(const vqk_weights *w, const Geom &g, int64_t N) {
     return size_t((N + rows - 1) / rows * rows) * size_t((g.NB + 3) / 4 * 4 * kBlock * g.D) * 2;
 }
 
-int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N,
-               void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st) {
+int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, bool deq,
+               int64_t N, void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st) {
     LinParams p;
     memset(&p, 0, sizeof p);
     p.codes = static_cast<const uint32_t *>(w->codes);
@@ -57,6 +57,7 @@ int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_typ
     p.y_type = y_type;
     p.N = int32_t(N);
     p.x_type = x_type;
+    p.deq = deq;
     const int xm = lin_x_mode(g.D, x_type, xf);
     const size_t fb = xm == kXBF16x || xm == kXF32x ? 0 : lin_frag_bytes(w, g, N);
     if (fb && ws && ws_bytes >= fb &&
