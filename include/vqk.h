@@ -181,8 +181,8 @@ int vqk_grouped_gemm(const vqk_weights *w, const void *x, int32_t x_type,
 /* ---- a11: dense large-N path, _decode_matmul (vq_dense.py:262-312) ---------
  * y[N, OUT] = x[N, IN] . W^T for E == 1. Up to 64 rows: W = fp16(cb * s) is
  * decoded straight into matrix-core operands (no workspace, x rounded to fp16
- * as the fused kernels take it). Above (and for shapes that path refuses): the reference's
- * decode-then-matmul, `xf @ w.T.astype(xf.dtype)` -- W is dequantised into the
+ * as the fused kernels take it). Above (and for shapes that path refuses, among them bf16 / fp32 x
+ * on rows that are not whole 32-code blocks): the reference's decode-then-matmul, `xf @ w.T.astype(xf.dtype)` -- W is dequantised into the
  * workspace panel by panel in x's arithmetic type and multiplied by libvqk's
  * matrix-core GEMM with fp32 accumulation: fp16 x against the bit-exact fp16
  * W, bf16 x against W rounded once to bf16, fp32 x through split bf16

@@ -190,3 +190,29 @@ def test_linear_rows_dead():
         x = torch.from_numpy(rng.standard_normal((N, m["IN"])).astype(np.float32)).cuda().half()
         y, ref = _apply(w, x), _apply(full, x)
         assert np.array_equal(y, ref) and not np.signbit(y[:, rt[0] < 0]).any()
+
+
+@pytest.mark.parametrize("d,K,packed,IN", [(4, 4096, True, 1088), (4, 256, False, 4160), (8, 4096, True, 1088),
+                                           (8, 65536, False, 4160)])
+def test_linear_ragged_past_fused_rows(d, K, packed, IN):
+    """33..64 rows of weight rows with a ragged last block at the default
+    options multiply in x's own arithmetic: fp32 x to 16 significant bits (two
+    bf16 parts: 2^-17 of each term, beside the fp32 sums), bf16 x beyond fp16's
+    range finite, against W rounded once to bf16; fp16 x against the decoded
+    weight."""
+    rng = np.random.default_rng(d + IN)
+    m = make_module(rng, 1, 70, IN, d, K, packed=packed)
+    w, keep = _desc(m)
+    for N in (33, 48, 64):
+        print(f"linear ragged d{d} K{K} {IN} N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda()
+        ref, bar = _ref(m, x, rounded=False, decoded=True)
+        bar = bar + bar / (IN * 2.0 ** -24) * 2.0 ** -17
+        assert (np.abs(_apply(w, x, fused=32) - ref) <= bar).all()
+        ref, bar = _ref(m, x, rounded=True, decoded=True)
+        assert (np.abs(_apply(w, x.half(), fused=32) - ref) <= bar).all()
+        big = (x * 1e6).bfloat16()
+        wb = vo.bf16_values(_weight(m, True).astype(np.float32)).astype(np.float64)
+        xb = big.double().cpu().numpy()
+        y = _apply(w, big, fused=32)
+        assert (np.abs(y - xb @ wb.T) <= np.abs(xb) @ np.abs(wb).T * (IN * 2.0 ** -24)).all()

@@ -859,7 +859,10 @@ int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type, int64_t 
     if ((rc = check_acts(x, x_type, y, y_type, N))) return rc;
     if (N < 0 || N > INT32_MAX) return set_error(VQK_EINVAL, "N=%lld", (long long)N);
     if (N == 0) return VQK_OK;
-    if (N <= kSegDenseMaxN && lin_ok(w, g, x, x_type, false, N))
+    // Ragged rows were never the segment kernel's: their bf16 / fp32 x keeps its
+    // own arithmetic below, which the few-row kernel's fp16 x would not.
+    if (N <= kSegDenseMaxN && (x_type == VQK_F16 || seg_fits(g, w, x)) &&
+        lin_ok(w, g, x, x_type, false, N))
         return launch_lin(w, g, x, x_type, false, true, N, y, y_type, workspace, ws_bytes, hipStream_t(stream));
     if (N <= kSegDenseMaxN && seg_fits(g, w, x)) {
         SegParams sp;
