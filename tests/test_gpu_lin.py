@@ -66,12 +66,12 @@ def _ref(m, x, rounded, decoded=False):
     return xv @ w.T, np.abs(xv) @ np.abs(w).T * (m["IN"] * 2.0 ** -24)
 
 
-# (d, K, packed, OUT, IN): more blocks per row than a GEMV wave holds; ragged
-# last blocks of every width class; OUT off the 16-row tile; a table in LDS,
-# partly in LDS, and not in LDS at all
+# (d, K, packed, OUT, IN): more blocks per row than a GEMV wave holds or ragged
+# last blocks, which this kernel takes at every size; OUT off the 16-row tile; a
+# table in LDS, partly in LDS, and not in LDS at all
 SHAPES = [
-    (2, 256, False, 100, 1088), (2, 1024, True, 33, 4224), (4, 256, False, 40, 1344),
-    (4, 4096, True, 130, 8448), (4, 8192, True, 17, 1088), (4, 65536, False, 48, 2048),
+    (2, 256, False, 100, 4160), (2, 1024, True, 33, 4224), (4, 256, False, 40, 1344),
+    (4, 4096, True, 130, 8448), (4, 8192, True, 17, 1088), (4, 65536, False, 48, 2112),
     (8, 4096, True, 65, 1088), (8, 16384, True, 40, 4160), (8, 65536, False, 33, 16640),
 ]
 
@@ -126,9 +126,10 @@ def test_linear_rows_scale_in_fp32(d, K, packed):
     """The scale multiplies a group's fp32 sum, not the fp16 entry: products of
     entry and scale above fp16's range (rows 0, 3, ...) and among its subnormals
     (rows 1, 4, ...) come out as exactly as the others, whatever the row count;
-    IN leaves the last superstep one block and half a block."""
+    IN leaves the last superstep one block, or one and half a block."""
     rng = np.random.default_rng(d + K)
-    m = make_module(rng, 1, 50, 64 * 33, d, K, packed=packed, cb_std=2.0)
+    IN = 64 * 65 if d == 2 else 64 * 33         # no fast GEMV: more than 64 blocks, or a ragged one
+    m = make_module(rng, 1, 50, IN, d, K, packed=packed, cb_std=2.0)
     m["scales"][0, 0::3] *= np.float16(40000)
     m["scales"][0, 1::3] *= np.float16(2.0 ** -12)
     m["codebook"][: K // 2] *= np.float16(2.0 ** -10)
@@ -142,6 +143,50 @@ def test_linear_rows_scale_in_fp32(d, K, packed):
             ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
             y = _apply(w, x)
             assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
+
+
+# (d, K, packed, OUT, IN, x, rows): both sides of each size from which the few-row
+# kernel takes over from the GEMV (20, 40, 70, 30, 90 and 40 million products)
+EDGES = [(2, 256, False, 1024, 2048, "f16", (9, 10)), (4, 4096, True, 1024, 4096, "bf16", (9, 10)),
+         (8, 4096, True, 2048, 2048, "f16", (16, 17)), (8, 16384, True, 1024, 2048, "f16", (14, 15)),
+         (8, 4096, True, 1024, 4096, "bf16", (2, 21, 22)), (8, 65536, False, 1024, 2048, "f32", (19, 20))]
+
+
+@pytest.mark.parametrize("d,K,packed,OUT,IN,dt,rows", EDGES)
+def test_linear_rows_at_the_gemv_edge(d, K, packed, OUT, IN, dt, rows):
+    """Rows on both sides of the size from which the few-row kernel runs in
+    place of the GEMV: one arithmetic, the same bar."""
+    rng = np.random.default_rng(d + K)
+    m = make_module(rng, 1, OUT, IN, d, K, packed=packed)
+    w, keep = _desc(m)
+    for N in rows:
+        print(f"linear edge d{d} K{K} {dt} N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda().to(DT[dt])
+        ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
+        assert (np.abs(_apply(w, x) - ref) <= bar).all(), N
+
+
+# both sides of each line between the segment kernel and the few-row kernel
+SEG_EDGES = [(2, 1024, True, 6400, 1024, (48, 49)), (4, 4096, True, 256, 1024, (40,)), (4, 4096, True, 256, 1536, (40,)),
+             (4, 1024, True, 8576, 2048, (33, 48, 49)), (4, 8192, True, 8576, 1536, (48, 49)), (4, 8192, True, 8192, 1024, (48, 64)),
+             (8, 4096, True, 16384, 3072, (16, 17, 33)), (8, 4096, True, 256, 2048, (8, 40)),
+             (8, 16384, True, 256, 2048, (32, 33)), (8, 65536, False, 8192, 1024, (48, 64))]
+
+
+@pytest.mark.parametrize("d,K,packed,OUT,IN,rows", SEG_EDGES)
+def test_linear_rows_at_the_segment_edge(d, K, packed, OUT, IN, rows):
+    """The same for the decoded-weight path (every row through vqk_dense_gemm):
+    the oracle on sampled columns, x rounded to fp16, W the dequant's fp16."""
+    rng = np.random.default_rng(d + K)
+    m = make_module(rng, 1, OUT, IN, d, K, packed=packed)
+    w, keep = _desc(m)
+    cols = rng.choice(OUT, min(OUT, 300), replace=False)
+    sub = dict(m, codes=m["codes"][:, cols], scales=m["scales"][:, cols], OUT=len(cols))
+    for N in rows:
+        print(f"linear segment edge d{d} K{K} {IN}->{OUT} N{N}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda()
+        ref, bar = _ref(sub, x, rounded=True, decoded=True)
+        assert (np.abs(_apply(w, x, fused=0)[:, cols] - ref) <= bar).all(), N
 
 
 def test_linear_rows_keep_x():

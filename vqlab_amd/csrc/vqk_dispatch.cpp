@@ -134,8 +134,8 @@ int vqk_linear_apply_scratch(const vqk_weights *w, int64_t N, const vqk_options 
     if (rc) return rc;
     Geom g;
     if ((rc = make_geom(w, &g))) return rc;
-    const size_t fb = lin_frag_bytes(w, g, N);
-    if (fb > *bytes) *bytes = fb;
+    if (!linear_fused(g, N, resolved(opt))) return vqk_dense_gemm_scratch(w, N, bytes);
+    *bytes = lin_frag_bytes(w, g, N);
     return VQK_OK;
 }
 

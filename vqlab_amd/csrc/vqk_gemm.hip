@@ -844,7 +844,8 @@ int vqk_dense_gemm_scratch(const vqk_weights *w, int64_t N, size_t *bytes) {
     if (rc) return rc;
     Geom g;
     if ((rc = make_geom(w, &g))) return rc;
-    const size_t fb = N <= kSegDenseMaxN ? lin_frag_bytes(w, g, N) : 0;
+    const bool lin = N <= kSegDenseMaxN && (!seg_fits_geom(g, w) || lin_beats_seg(g, N));
+    const size_t fb = lin ? lin_frag_bytes(w, g, N) : 0;
     if (fb > *bytes) *bytes = fb;
     return VQK_OK;
 }
@@ -861,10 +862,11 @@ int vqk_dense_gemm(const vqk_weights *w, const void *x, int32_t x_type, int64_t 
     if (N == 0) return VQK_OK;
     // Ragged rows were never the segment kernel's: their bf16 / fp32 x keeps its
     // own arithmetic below, which the few-row kernel's fp16 x would not.
-    if (N <= kSegDenseMaxN && (x_type == VQK_F16 || seg_fits(g, w, x)) &&
+    const bool seg = N <= kSegDenseMaxN && seg_fits(g, w, x);
+    if (N <= kSegDenseMaxN && (seg ? lin_beats_seg(g, N) : x_type == VQK_F16) &&
         lin_ok(w, g, x, x_type, false, N))
         return launch_lin(w, g, x, x_type, false, true, N, y, y_type, workspace, ws_bytes, hipStream_t(stream));
-    if (N <= kSegDenseMaxN && seg_fits(g, w, x)) {
+    if (seg) {
         SegParams sp;
         fill_seg(w, g, &sp);
         sp.x = x;

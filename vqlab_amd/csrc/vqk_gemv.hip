@@ -65,7 +65,8 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
     // wide x at d=4: fast instances for the unpacked widths, else the generic kernel
     const bool fast_x = !xf || g.D == 8 || gemv_fast_d4x_has(g.BITS);
     const bool fast = g.fast_ok && fast_x && gemv_fast_lds(g, xf) <= size_t(kLdsBytes);
-    if (!eidx && (N > 1 || !fast) && lin_ok(w, g, x, x_type, xf, N))
+    if (!eidx && (!fast || (N > 1 && lin_beats_gemv(g, xf && x_type != VQK_F16, N))) &&
+        lin_ok(w, g, x, x_type, xf, N))
         return launch_lin(w, g, x, x_type, xf, false, N, y, y_type, ws, ws_bytes, st);
     GemvParams p;
     gemv_fill_params(w, g, &p);

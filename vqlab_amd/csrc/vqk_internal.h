@@ -23,6 +23,10 @@ int launch_gemv(const vqk_weights *w, const void *x, int32_t x_type, int64_t T,
 // The few-row linear kernel (vqk_lin.h) for N rows of one linear: whether it
 // takes the module and x (xf: x unrounded, VQK_X_KEEP), and its launch.
 bool lin_ok(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, int64_t N);
+// ... and whether it is the faster one for a module that the fast GEMV (wide: x
+// enters as fp32) or the segment kernel takes too.
+bool lin_beats_gemv(const Geom &g, bool wide, int64_t N);
+bool lin_beats_seg(const Geom &g, int64_t N);
 int launch_lin(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, bool xf, bool deq,
                int64_t N, void *y, int32_t y_type, void *ws, size_t ws_bytes, hipStream_t st);
 

@@ -38,7 +38,7 @@
 // Measured (MI355X, us per call, this kernel / the GEMV or, for 64 rows, the
 // segment kernel; bf16 x):
 //   5120 -> 17408, d4 K4096:  8 rows 28 / 102, 17 rows 35 / 204, 64 rows 51 / 68
-//   17408 -> 5120, d4 K4096:  1 row 25 / 1719, 17 rows 37 / 3242 (generic GEMV)
+//   17408 -> 5120, d4 K4096:  1 row 25 / 1719, 17 rows 36 / 3242 (generic GEMV)
 //   5120 -> 17408, d8 K65536: 8 rows 77 / 411, 17 rows 134 / 831 (fp32 products)
 #pragma once
 
@@ -488,8 +488,8 @@ __global__ void __launch_bounds__(256) k_lin_frag(const void *x, int x_type, int
 }
 
 // Rows up to which the direct loads always serve: each row of x adds its cache
-// lines to every operand load (5120 -> 17408, d4 K4096: 4 rows 29 us in place,
-// 8 rows 38 in place and 31 with the copy).
+// lines to every operand load (5120 -> 17408, d4 K4096: 4 rows 28 us in place,
+// 8 rows 33 in place and 26 with the copy).
 constexpr int kLinDirectRows = 4;
 
 // 16-row tiles of x sharing one decode, for N rows in operand order
@@ -505,9 +505,9 @@ inline int lin_groups(const LinParams &p, int l) {
 // superstep) the one whose busiest CU walks the fewest supersteps --
 // workgroups per CU, rounded up, times supersteps per wave, rounded up; the
 // fewest slices of equals (each row group reads all of x). It picks the
-// measured best of all four at 5120 -> 17408 (4 slices: 20 rows 36 us against
-// 39 / 39 / 37), 17408 -> 5120 (4: 36 against 111 / 60 / 38) and 8192 -> 8192
-// (4: 26 against 55 / 32 / 27), d4 K4096.
+// measured best of all four at 5120 -> 17408 (4 slices: 20 rows 35 us against
+// 39 / 40 / 38), 17408 -> 5120 (4: 36 against 110 / 59 / 38) and 8192 -> 8192
+// (4: 21 against 55 / 32 / 23), d4 K4096.
 inline int lin_slices(const LinParams &p, int tiles) {
     const int64_t nss = (p.NB + 3) / 4;
     int best = 0;
@@ -529,8 +529,8 @@ int go_lin_tile(LinParams p, hipStream_t st) {
 
 // x in place: one 16-row tile; in operand order: tiles of 16, 32 or 64 rows.
 // One 16-row weight tile per wave: two, sharing each x operand, halve the
-// waves and ran 1.3-1.7x slower at every shape above (20 rows of 5120 ->
-// 17408: 61 us against 36).
+// waves and, in this kernel's first form, ran 1.3-1.7x slower at every shape
+// above (20 rows of 5120 -> 17408: 61 us against 36).
 template <int D, int BITS, int GPB, int XM, bool DEQ>
 int go_lin_mode(const LinParams &p, hipStream_t st) {
     if constexpr (XM != kXFrag) {

@@ -24,9 +24,52 @@ bool lin_ok(const vqk_weights *w, const Geom &g, const void *x, int32_t x_type, 
            N <= (int64_t(1) << 31) / (g.IN * act_size(x_type));      // x as one buffer of <= 2 GB
 }
 
+// Against the GEMV, which decodes every weight once per row but has no K loop
+// to start and end: the products from which the few-row kernel is ahead, by
+// what bounds the GEMV there. us per call, GEMV / this kernel (MI355X, graph
+// replays), the last size that stays and the first that goes:
+//   d2            20e6  4096 -> 1024: 4 rows 6.0 / 7.0, 5 rows 7.0 / 7.0
+//   d4            40e6  4096 -> 4096, K4096: 2 rows 7.6 / 7.6, 3 rows 10 / 7.6
+//   d8 fp16 x     70e6  4096 -> 4096, K4096: 4 rows 12 / 9; 30e6 with a table
+//                       beyond LDS: 4096 -> 4096, K16384: 2 rows 12 / 13
+//   d8 wide x     90e6  4096 -> 4096, K4096: 4 rows 15.5 / 17, 8 rows 25 / 17,
+//                       and more than two rows (5120 -> 17408: 2 rows 53 / 62);
+//                       40e6 with a table beyond LDS
+// Over 14 sizes from 1024 -> 512 to 5120 -> 17408 and 2..32 rows of 9 formats
+// the rule is within 20 % of the better of the two, most often with it; always
+// taking this kernel cost up to 3x (1024 -> 1024, d8 K4096: 5.5 against 16).
+bool lin_beats_gemv(const Geom &g, bool wide, int64_t N) {
+    const bool lds = cb_in_lds(g.D, g.BITS);
+    if (wide && lds && N <= 2) return false;
+    const int64_t from = g.D == 2 ? 20000000 : g.D == 4 ? 40000000
+                       : lds ? (wide ? 90000000 : 70000000) : (wide ? 40000000 : 30000000);
+    return N * g.OUT >= (from + g.IN - 1) / g.IN;
+}
+
+// Against the segment kernel, which decodes once per 16 rows with one workgroup
+// to 128 weight rows and no K slices: it stays ahead over few supersteps, where
+// the slices have nothing to share, and where its workgroups fill the chip in
+// one round while this kernel's 64-row tile is part empty. us, segment / this:
+//   d4 K4096: 1024 -> 4096 (2 supersteps) 33 rows 9.0 / 9.5; 2048 -> 2048 (4) 14 / 10;
+//             5120 -> 17408 (136 workgroups to 16 rows) 33 rows 39 / 48, 49 rows 61 / 48
+//   d4 K8192 (one workgroup to a CU): 3072 -> 9216 (216 workgroups) 33 rows 20 / 23
+//   d8 K4096: 2048 -> 2048 (2) 33 rows 11 / 14; 5120 -> 17408 16 rows 21 / 23, 33 rows 43 / 50
+//   d8 K16384, K65536: 2048 -> 2048 (2) 8 rows 19 / 14, 64 rows 18 / 22
+bool lin_beats_seg(const Geom &g, int64_t N) {
+    const int64_t nss = (g.NB + 3) / 4, wgs = (g.OUT + 127) / 128 * ((N + 15) / 16);
+    const bool part_empty = N > 32 && N <= 48 && wgs >= 200;
+    if (g.D == 2) return !(part_empty && nss <= 4);
+    if (g.D == 8 && N <= 16 && wgs >= 128) return false;
+    // two of the segment kernel's workgroups to a CU, or a d8 table in LDS
+    if (cb_in_lds(g.D, g.BITS) && (g.D == 8 || (int64_t(1) << g.BITS) * g.D * 2 <= 32 * 1024))
+        return nss > 2 && !part_empty;
+    if (g.D == 4 && part_empty && wgs <= 256) return false;
+    return nss > (N > 32 || g.D == 4 ? 2 : 1) || wgs >= 256;
+}
+
 // The copy pays from about 2^28 products on: below, its launch costs more (3 us
 // on the GPU, 5 for a caller that waits on the host) than the direct loads
-// lose (0.3 us per million weights and 16 rows: 26 us at 5120 -> 17408).
+// lose (0.2 us per million weights and 16 rows: 17 us at 5120 -> 17408).
 constexpr int64_t kLinFragWork = int64_t(1) << 28;
 
 size_t lin_frag_bytes(const vqk_weights *w, const Geom &g, int64_t N) {
