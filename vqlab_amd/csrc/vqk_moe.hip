@@ -1824,6 +1824,8 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         int r = hip_status(hipEventRecord(ss->e[i], from), "hipEventRecord");
         return r ? r : hip_status(hipStreamWaitEvent(to, ss->e[i], 0), "hipStreamWaitEvent");
     };
+    // where only the shared expert runs on the second stream: nothing without one
+    auto fork = [&](int i, hipStream_t from, hipStream_t to) { return p.shared ? link(i, from, to) : VQK_OK; };
     const int wide = N >= kMoeWideMinPairs * p.E ? wide_tile_rows(m->gate, m->up, m->down, N) : 0;
     if (wide && (!p.shared || wide_tile_rows(m->sh_gate, m->sh_up, m->sh_down, T))) {
         // Many rows per expert. x as fp16 rows (where yd goes later) unless it
@@ -1835,7 +1837,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
             if ((rc = launch_x_half(p.x, p.x_type, T * p.H, xc, st))) return rc;
             xh = xc;
         }
-        if ((rc = link(0, st, sb))) return rc;
+        if ((rc = fork(0, st, sb))) return rc;
         if (p.shared) {
             const WideCall cs{xh, 1, sgg, VQK_F16, T, 0};
             if ((rc = wide_run(m->sh_gate, m->sh_up, cs, nullptr, sb))) return rc;
@@ -1845,14 +1847,14 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         if ((rc = seg_sort(reinterpret_cast<const uint32_t *>(p.ids), N, p.E, wide, sort, st))) return rc;
         const WideCall c{xh, k, g, VQK_F16, N, wide};
         if ((rc = wide_run(m->gate, m->up, c, sort, st))) return rc;
-        if ((rc = link(1, sb, st))) return rc;                    // down overwrites xh
+        if ((rc = fork(1, sb, st))) return rc;                    // down overwrites xh
         if (p.shared) {
             const WideCall ds{reinterpret_cast<const uint16_t *>(sgg), 1, ysh, VQK_F32, T, 0};
             if ((rc = wide_run(m->sh_down, nullptr, ds, nullptr, sb))) return rc;
         }
         const WideCall d{reinterpret_cast<const uint16_t *>(g), 0, yd, VQK_F32, N, wide};
         if ((rc = wide_run(m->down, nullptr, d, sort, st))) return rc;
-        if ((rc = link(3, sb, st))) return rc;
+        if ((rc = fork(3, sb, st))) return rc;
         hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
                            p, static_cast<const float *>(yd), static_cast<const float *>(ysh), static_cast<const float *>(nullptr), static_cast<const float *>(nullptr));
         return hip_status(hipGetLastError(), "combine launch");
@@ -1867,7 +1869,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         uint16_t *hs = reinterpret_cast<uint16_t *>(ws + pl.lay.hs), *hsh = reinterpret_cast<uint16_t *>(ws + pl.lay.hsh);
         float *y1 = reinterpret_cast<float *>(ws + pl.lay.y1), *ysh1 = reinterpret_cast<float *>(ws + pl.lay.ysh1);
         if ((rc = launch_x_split(p.x, p.x_type, T * p.H, xh, st))) return rc;
-        if ((rc = link(0, st, sb))) return rc;
+        if ((rc = fork(0, st, sb))) return rc;
         if (p.shared) {
             float *sg1 = sgg + T * p.I, *su1 = sgu + T * p.I;
             const HalfCall cs{xh, 1, {{sgg, sg1}, {sgu, su1}}, true, T};
@@ -1883,7 +1885,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         const HalfCall c{xh, k, {{g, g1}, {u, u1}}, true, N};
         if ((rc = half_run(m->gate, m->up, c, sort, st))) return rc;
         if ((rc = launch_swiglu_split(g, g1, u, u1, N * p.I, hs, st))) return rc;
-        if ((rc = link(1, sb, st))) return rc;                    // down overwrites xh
+        if ((rc = fork(1, sb, st))) return rc;                    // down overwrites xh
         const HalfCall d{hs, 0, {{yd, y1}, {}}, false, N};
         if ((rc = half_run(m->down, nullptr, d, sort, st))) return rc;
         hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
