@@ -50,6 +50,18 @@ CASES = [
     (8, 256, 512, 8, 1024, 2, 64, False, 0.0),
     (3, 512, 256, 4, 8192, 2, 200, False, 0.3),
     (160, 256, 256, 8, 2048, 4, 80, False, 0.0),
+    # the shared expert as wide tiles too (512 rows and more)
+    (4, 512, 384, 4, 1024, 2, 520, True, 0.0),
+    (4, 768, 256, 8, 4096, 2, 530, True, 0.2),
+    # both sides of the pairs per expert from which wide tiles run: three over a
+    # small table beside a shared expert, ten beside it over few experts and
+    # where few workgroups walk a long row (four over a 64 KB table)
+    (128, 256, 256, 4, 256, 2, 191, True, 0.0),
+    (128, 256, 256, 4, 256, 2, 192, True, 0.0),
+    (16, 256, 256, 4, 1024, 2, 79, True, 0.0),
+    (16, 256, 256, 4, 1024, 2, 80, True, 0.0),
+    (32, 2304, 256, 4, 8192, 2, 63, False, 0.2),
+    (32, 2304, 256, 4, 8192, 2, 64, False, 0.2),
 ]
 
 

@@ -657,6 +657,34 @@ int wide_tile_rows(const vqk_weights *gate, const vqk_weights *up, const vqk_wei
     return 32 * (n1 < n2 ? n1 : n2);
 }
 
+// From one pair per expert on, except where the 16-row kernel is ahead for some
+// rows more: over d4 tables of up to 32 KB (two of its workgroups to a CU) with
+// many weights and a down projection of long rows, beside a shared expert (the wide form then pays for a second
+// stream too), or where few workgroups walk long rows. us per layer as a graph
+// replay, 16-row / wide (MI355X):
+//   256 experts of 2048 x 512,  d4 K4096: 32 tokens 109 / 127, 64 tokens 144 / 136
+//   256 experts of 2048 x 1024, d4 K4096: 32 tokens 186 / 232, 96 tokens 251 / 245
+//   256 experts of 4096 x 256,  d4 K4096: 32 tokens 137 / 122
+//   64 experts of 4096 x 256,   d4 K4096: 16 tokens 83 / 94, 64 tokens 90 / 95
+//   64 experts of 2048 x 512 and a shared one, d4 K4096: 16 tokens 69 / 84,
+//                                         64 tokens 77 / 84, 96 tokens 91 / 86
+//   256 experts of 2048 x 512,  d8 K4096: 64 tokens 179 / 113
+// Without a shared expert a call of its own (no graph) is 13 to 40 us longer on
+// the 16-row kernels, whose up projection is on the second stream.
+bool wide_pays(const vqk_weights *gate, bool shared, int64_t N) {
+    Geom g;
+    if (make_geom(gate, &g)) return false;
+    int64_t pairs = 1;
+    if (g.D == 4) {
+        const bool small = (int64_t(1) << g.BITS) * g.D * 2 <= 32 * 1024;
+        const bool few = g.E * ((g.OUT + 255) / 256) < 128 && g.IN > 2048;
+        if (few || (shared && g.E < 128)) pairs = small ? 10 : 4;
+        else if (small && shared) pairs = 3;
+        else if (small && g.OUT >= 512 && g.E * g.OUT >= (int64_t(1) << 28) / g.IN) pairs = 2;
+    }
+    return N >= pairs * g.E;
+}
+
 static void fill_wide(const vqk_weights *w, const Geom &g, WideMod *m) {
     m->codes = static_cast<const uint32_t *>(w->codes);
     m->row_words = g.row_words;

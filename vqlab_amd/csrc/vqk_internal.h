@@ -94,6 +94,9 @@ struct WideCall {
 // Rows per tile to sort a routing of N pairs into for the projections of a layer,
 // or 0 when the wide kernel does not take them.
 int wide_tile_rows(const vqk_weights *gate, const vqk_weights *up, const vqk_weights *down, int64_t N);
+// Whether the wide kernel is the faster one for N pairs over gate's experts (and
+// a shared one).
+bool wide_pays(const vqk_weights *gate, bool shared, int64_t N);
 // `up`: with it, SwiGLU of (w, up). sort_ws: the sorted routing, or NULL for
 // dense rows of one expert.
 int wide_run(const vqk_weights *w, const vqk_weights *up, const WideCall &c, const void *sort_ws,

@@ -39,12 +39,13 @@ constexpr int kMaxTopK = 64;
 // config-3 layer, T = 16 -> 160 pairs over 512 experts: 698 us sliced GEMV
 // against 745 us grouped; T = 64: 2583 us against 1588 us)
 constexpr int64_t kMoeGroupedMinPairs = 64;
-// pairs per expert from which the grouped projections run as wide tiles
-// (vqk_wide.h; tables of up to 64 KB): level with the 16-row kernel there
-// (256 experts of 2048 x 512, d4 K4096: 33 tokens 151 us against 157) and ahead
-// of it from then on (256 tokens 168 / 198, 2048 tokens 272 / 704; 160 experts
-// of 2560 x 1024, d8 K4096: 128 tokens 204 / 272, 2048 tokens 624 / 2276)
-constexpr int64_t kMoeWideMinPairs = 1;
+// Token rows from which the shared expert of a layer with wide tiles runs as
+// wide tiles too: they are few long workgroups (12 for 512 rows of an expert of
+// 2048 x 512), where the 16-row kernels split K. us per layer as a graph replay,
+// 16-row / wide shared expert (MI355X): 256 experts of 2048 x 512, d4 K4096, 256
+// tokens 170 / 192, 768 tokens 229 / 229, 2048 tokens 336 / 311; 64 experts of
+// 4096 x 1024, d8 K4096, 128 tokens 150 / 169, 512 tokens 214 / 201.
+constexpr int64_t kMoeWideSharedRows = 512;
 
 struct MoeW {            // one projection of the layer, as the kernels see it
     const uint32_t *codes;
@@ -1826,19 +1827,40 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
     };
     // where only the shared expert runs on the second stream: nothing without one
     auto fork = [&](int i, hipStream_t from, hipStream_t to) { return p.shared ? link(i, from, to) : VQK_OK; };
-    const int wide = N >= kMoeWideMinPairs * p.E ? wide_tile_rows(m->gate, m->up, m->down, N) : 0;
-    if (wide && (!p.shared || wide_tile_rows(m->sh_gate, m->sh_up, m->sh_down, T))) {
+    // The shared expert on the 16-row kernels is one expert over T rows: its gate
+    // / up launches alone would fill few CUs, so they split K (fp32 partials that
+    // the down launch adds in a fixed order as it stages its input).
+    const int ks = p.shared ? seg_ksplit(m->sh_gate, T) : 1;
+    auto shared_seg_up = [&](hipStream_t s) {
+        SegCall cs{p.x, p.x_type, nullptr, nullptr, 1, sgg, VQK_F32, T, 0, ks};
+        int r = seg_run(m->sh_gate, cs, nullptr, s);
+        cs.y = sgu;
+        return r ? r : seg_run(m->sh_up, cs, nullptr, s);
+    };
+    auto shared_seg_down = [&](hipStream_t s) {
+        SegCall ds{nullptr, VQK_F32, sgg, sgu, 1, ysh, VQK_F32, T, 0, 0, ks};
+        return seg_run(m->sh_down, ds, nullptr, s);
+    };
+    const int wide = wide_pays(m->gate, p.shared, N) ? wide_tile_rows(m->gate, m->up, m->down, N) : 0;
+    const bool sh_wide = p.shared && T >= kMoeWideSharedRows &&
+                         wide_tile_rows(m->sh_gate, m->sh_up, m->sh_down, T);
+    if (wide) {
         // Many rows per expert. x as fp16 rows (where yd goes later) unless it
         // is; gate and up at once into fp16 SwiGLU rows in sorted order (in g);
-        // down over those. The shared expert is the same over the token rows.
+        // down over those. The shared expert over the token rows is the same, or
+        // (under kMoeWideSharedRows) the 16-row kernels.
+        if (p.shared && !sh_wide) {
+            if ((rc = link(0, st, sb))) return rc;
+            if ((rc = shared_seg_up(sb))) return rc;
+        }
         const uint16_t *xh = static_cast<const uint16_t *>(p.x);
         if (p.x_type != VQK_F16) {
             uint16_t *xc = reinterpret_cast<uint16_t *>(yd);
             if ((rc = launch_x_half(p.x, p.x_type, T * p.H, xc, st))) return rc;
             xh = xc;
         }
-        if ((rc = fork(0, st, sb))) return rc;
-        if (p.shared) {
+        if (sh_wide) {
+            if ((rc = link(0, st, sb))) return rc;
             const WideCall cs{xh, 1, sgg, VQK_F16, T, 0};
             if ((rc = wide_run(m->sh_gate, m->sh_up, cs, nullptr, sb))) return rc;
         }
@@ -1847,10 +1869,12 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
         if ((rc = seg_sort(reinterpret_cast<const uint32_t *>(p.ids), N, p.E, wide, sort, st))) return rc;
         const WideCall c{xh, k, g, VQK_F16, N, wide};
         if ((rc = wide_run(m->gate, m->up, c, sort, st))) return rc;
-        if ((rc = fork(1, sb, st))) return rc;                    // down overwrites xh
-        if (p.shared) {
+        if (sh_wide) {
+            if ((rc = link(1, sb, st))) return rc;                // down overwrites xh
             const WideCall ds{reinterpret_cast<const uint16_t *>(sgg), 1, ysh, VQK_F32, T, 0};
             if ((rc = wide_run(m->sh_down, nullptr, ds, nullptr, sb))) return rc;
+        } else if (p.shared && (rc = shared_seg_down(sb))) {
+            return rc;
         }
         const WideCall d{reinterpret_cast<const uint16_t *>(g), 0, yd, VQK_F32, N, wide};
         if ((rc = wide_run(m->down, nullptr, d, sort, st))) return rc;
@@ -1893,17 +1917,8 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
                            static_cast<const float *>(y1), p.shared ? static_cast<const float *>(ysh1) : none);
         return hip_status(hipGetLastError(), "combine launch");
     }
-    // the shared expert is one expert over T rows: its gate / up launches
-    // alone would fill few CUs, so they split K (fp32 partials that the down
-    // launch adds in a fixed order as it stages its input)
-    const int ks = p.shared ? seg_ksplit(m->sh_gate, T) : 1;
     if ((rc = link(0, st, sb))) return rc;
-    if (p.shared) {
-        SegCall cs{p.x, p.x_type, nullptr, nullptr, 1, sgg, VQK_F32, T, 0, ks};
-        if ((rc = seg_run(m->sh_gate, cs, nullptr, sb))) return rc;
-        cs.y = sgu;
-        if ((rc = seg_run(m->sh_up, cs, nullptr, sb))) return rc;
-    }
+    if (p.shared && (rc = shared_seg_up(sb))) return rc;
     hipLaunchKernelGGL(k_route_tokens, dim3(unsigned(T)), dim3(kWave), 0, st, p);
     if ((rc = hip_status(hipGetLastError(), "routing launch"))) return rc;
     // one sort for the three routed projections: its tile rows must suit
@@ -1919,10 +1934,7 @@ static int launch_moe_grouped(const vqk_moe_desc *m, const MoePlan &pl, uint8_t 
     if ((rc = link(2, sb, st))) return rc;
     SegCall d{nullptr, VQK_F32, g, u, 1, yd, VQK_F32, N, tok};
     if ((rc = seg_run(m->down, d, sort, st))) return rc;
-    if (p.shared) {
-        SegCall ds{nullptr, VQK_F32, sgg, sgu, 1, ysh, VQK_F32, T, 0, 0, ks};
-        if ((rc = seg_run(m->sh_down, ds, nullptr, sb))) return rc;
-    }
+    if (p.shared && (rc = shared_seg_down(sb))) return rc;
     if ((rc = link(3, sb, st))) return rc;
     hipLaunchKernelGGL(k_moe_combine, dim3(unsigned((p.H + 1023) / 1024), unsigned(T)), dim3(256), 0, st,
                        p, static_cast<const float *>(yd), static_cast<const float *>(ysh), static_cast<const float *>(nullptr), static_cast<const float *>(nullptr));
