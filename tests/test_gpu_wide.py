@@ -117,6 +117,36 @@ def test_moe_many_rows_not_finite():
     assert torch.equal(z[keep], y[keep]) and not torch.isfinite(z[7]).any()
 
 
+@pytest.mark.parametrize("d,K", [(4, 1024), (8, 1024), (8, 16384)])
+def test_moe_weight_beyond_fp16(d, K):
+    """A weight that overflows fp16 (row 5 of every expert's down projection, one
+    column) makes its output infinite, with the sign of what it multiplies, and
+    changes no other; with an odd block count, whose last superstep has a lane
+    group without a block (d8 16384: the half-entry kernel, same rule)."""
+    print(f"moe weight beyond fp16 d{d} K{K}", flush=True)
+    rng = np.random.default_rng(d)
+    E, H, I, k, T = 4, 512, 32 * d * (1 if d == 8 else 3), 2, 100
+    blk, ms, _, _ = _block(rng, E, H, I, d, K, k)
+    m = ms["down"]
+    m["codebook"][0] = 0
+    m["codebook"][0, 0] = 2.0
+    m["codes"][:, 5, -I // d:] = np.maximum(m["codes"][:, 5, -I // d:], 1)
+    m["codes"][:, 5, -1] = 0
+    m["scales"][:, 5, -1] = 60000.0
+    m["stored"] = vo.pack(m["codes"], m["pack_bits"])
+    blk.switch_mlp.down_proj = _lin(m, False)
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).cuda().half()
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    y = blk(x, torch.from_numpy(logits).cuda()).double().cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = _oracle(x, logits, ms, k, {})
+    same = ~np.isnan(ref[:, 5])                     # both experts' terms of one sign
+    assert np.isinf(ref[same, 5]).all() and same.mean() > 0.3
+    assert np.array_equal(y[same, 5], ref[same, 5]) and np.isnan(y[~same, 5]).all()
+    rest = [r for r in range(H) if r != 5]
+    assert_close(y[:, rest], ref[:, rest], what="beside a weight beyond fp16")
+
+
 @pytest.mark.parametrize("N", [24 * 1024, 24 * 1024 + 8])
 def test_sort_past_its_lds(N):
     """The pair order staged in LDS at its limit, and in place past it."""

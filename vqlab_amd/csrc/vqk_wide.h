@@ -170,6 +170,15 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
         }
     };
 
+    // a lane group without a block multiplies the zeros of its x by a weight of
+    // zero: the last block's again could be infinite
+    auto drop_scales = [&](int sb, uint16_t (&s)[NM][GPB]) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int g = 0; g < GPB; ++g) s[m][g] = 2 * sb + lg < p.NB ? s[m][g] : uint16_t(0);
+    };
+
     f32x16w acc[NM][NT];
     auto clear = [&]() {
 #pragma unroll
@@ -274,6 +283,7 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
 #pragma unroll
     for (int c = 0; c < NBUF - 1; ++c) copy_next(c);
     load_w(rw, 0, w, sc);
+    drop_scales(0, sc);
     clear();
     wait_vmem();                                // the tables and the first chunks
     __syncthreads();
@@ -314,6 +324,7 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
 #pragma unroll
                 for (int g = 0; g < GPB; ++g) sc[m][g] = sn[m][g];
             }
+            drop_scales(last ? 0 : sb + 1, sc);
         }
         store(rw);
         clear();
