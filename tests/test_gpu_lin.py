@@ -21,7 +21,9 @@ def _desc(m, row_table=None, sz=None):
     from vqlab_amd import _torch as Tt
     keep = []
     if sz is not None:
-        codes = torch.from_numpy(np.ascontiguousarray(sz["sz_codes"]).view(np.int32)).cuda()
+        st = np.ascontiguousarray(sz["sz_codes"])
+        signed = {4: np.int32, 2: np.int16, 1: np.uint8}[st.itemsize]
+        codes = torch.from_numpy(st.view(signed)).cuda()
         scales = torch.from_numpy(sz["sz_scales"]).cuda()
         cb = torch.from_numpy(m["codebook"]).cuda()
         rt = torch.from_numpy(row_table).cuda()
@@ -86,38 +88,50 @@ def test_linear_rows(d, K, packed, OUT, IN, dt):
         print(f"linear rows d{d} K{K} {IN}->{OUT} {dt} N{N}", flush=True)
         x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda().to(DT[dt])
         ref, bar = _ref(m, x, rounded=d != 8 or dt == "f16")
-        for scratch in (True, False):
-            y = _apply(w, x, scratch)
-            assert (np.abs(y - ref) <= bar).all(), (N, scratch, np.abs(y - ref).max(), bar.min())
+        y = _apply(w, x)
+        assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
 
 
-@pytest.mark.parametrize("d,K,packed", [(2, 1024, True), (4, 4096, True), (8, 16384, True),
-                                        (8, 65536, False)])
-def test_linear_rows_operand_order(d, K, packed):
-    """Shapes whose x is copied into operand order (2^28 products and more),
-    with a ragged last block and an odd OUT, at the edges of the row tiles: the
-    oracle on sampled columns; one row with an infinite value stays alone."""
+@pytest.mark.parametrize("d,K,packed,IN", [
+    (2, 1024, True, 4160), (2, 256, False, 4096), (4, 4096, True, 4160), (4, 1024, True, 4096),
+    (4, 65536, False, 4096), (8, 16384, True, 4160), (8, 4096, True, 4096), (8, 65536, False, 4160)])
+def test_linear_rows_operand_order(d, K, packed, IN):
+    """Shapes whose x is copied into operand order (2^28 products and more), with
+    a ragged last block or whole supersteps, an odd OUT and dead rows, at the
+    edges of the row tiles, against the oracle on sampled columns -- as without
+    scratch, where x is read in place; an infinite and a NaN value of x stay in
+    their rows."""
     from vqlab_amd import _lib as L
     rng = np.random.default_rng(d + K)
-    m = make_module(rng, 1, 13001, 4160, d, K, packed=packed)
-    w, keep = _desc(m)
-    cols = np.unique(np.concatenate([rng.choice(m["OUT"], 150, replace=False),
-                                     [0, 15, 16, 12999, 13000]]))
+    m = make_module(rng, 1, 13201, IN, d, K, packed=packed, dead_frac=0.02)
+    sz, rt = skipzero(m)
+    w, keep = _desc(m, rt, sz)
+    cols = np.unique(np.concatenate([rng.choice(m["OUT"], 150, replace=False), [0, 15, 16, 13199, 13200]]))
     sub = dict(m, codes=m["codes"][:, cols], scales=m["scales"][:, cols], OUT=len(cols))
-    for N in (5, 16, 17, 32, 33, 64):
-        print(f"linear operand order d{d} K{K} N{N}", flush=True)
+    for N in (5, 16, 17, 32, 33, 49, 64):
+        print(f"linear operand order d{d} K{K} {IN} N{N}", flush=True)
         o, ws = L.options(dense_fused_max_n=64), ctypes.c_size_t()
         L.check(L.lib().vqk_linear_apply_scratch(ctypes.byref(w), N, ctypes.byref(o), ctypes.byref(ws)))
         assert ws.value > 0
         x = torch.from_numpy(rng.standard_normal((N, m["IN"])).astype(np.float32)).cuda().half()
-        ref, bar = _ref(sub, x, rounded=True)
+        for fused in (64, 0):                       # scales in fp32, and the decoded weight
+            if fused == 0 and N <= 32:
+                continue
+            ref, bar = _ref(sub, x, rounded=True, decoded=fused == 0)
+            for scratch in (True, False):
+                if fused == 0 and not scratch and m["IN"] % (32 * d):
+                    continue                        # the ragged dense GEMM's own workspace
+                y = _apply(w, x, scratch, fused)[:, cols]
+                assert (np.abs(y - ref) <= bar).all(), (N, fused, scratch, np.abs(y - ref).max(), bar.min())
+                assert not np.signbit(y[:, rt[0][cols] < 0]).any()
         y = _apply(w, x)[:, cols]
-        assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
-        if d != 8:                              # bf16 / fp32 rounded on the way
+        if d != 8:                                  # bf16 / fp32 rounded on the way
             assert np.array_equal(_apply(w, x.float())[:, cols], y)
-        x[1, 7] = float("inf")
+        x[1, 7], x[3, IN - 1] = float("inf"), float("nan")
         y = _apply(w, x)
-        assert np.isfinite(y[[0] + list(range(2, N))]).all() and not np.isfinite(y[1]).any()
+        live = rt[0] >= 0
+        assert np.isfinite(y[[0, 2] + list(range(4, N))]).all()
+        assert not np.isfinite(y[1][live]).any() and np.isnan(y[3][live]).all()
 
 
 @pytest.mark.parametrize("d,K,packed", [(2, 1024, True), (4, 4096, True), (8, 4096, True),
@@ -216,11 +230,10 @@ def test_linear_rows_not_finite(d, K, IN):
         print(f"linear not finite d{d} N{N}", flush=True)
         x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda()
         x[1, 0], x[2, 3] = float("inf"), float("nan")
-        for scratch in (True, False):
-            y = _apply(w, x.half(), scratch)
-            assert np.isfinite(y[[0] + list(range(3, N))]).all()
-            w0 = vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64)[:, 0]
-            assert np.array_equal(y[1][w0 != 0], np.sign(w0[w0 != 0]) * np.inf) and np.isnan(y[2]).all()
+        y = _apply(w, x.half())
+        assert np.isfinite(y[[0] + list(range(3, N))]).all()
+        w0 = vo.dequant(m["codes"][0], m["codebook"], m["scales"][0], 64)[:, 0]
+        assert np.array_equal(y[1][w0 != 0], np.sign(w0[w0 != 0]) * np.inf) and np.isnan(y[2]).all()
 
 
 def test_linear_rows_dead():

@@ -87,6 +87,42 @@ def test_moe_many_rows(case, dt):
     assert_close(y.float().cpu().numpy(), ref, what=f"moe many rows {case}")
 
 
+# E, H, I, d, K, k, T, shared, dead: enough experts that a workgroup walks several
+# 256-row blocks of its tile -- two of three (H 768) and four of nine (H 2304) in
+# down, the last workgroup fewer; two of three in gate and up (I 768)
+BLOCK_CASES = [
+    (256, 768, 128, 4, 1024, 2, 280, False, 0.0),
+    (256, 2304, 128, 4, 4096, 2, 280, False, 0.2),
+    (256, 768, 256, 8, 2048, 2, 200, True, 0.2),
+    (256, 256, 768, 8, 1024, 2, 150, False, 0.2),
+    (256, 512, 768, 4, 8192, 2, 260, False, 0.0),
+]
+
+
+@pytest.mark.parametrize("case", BLOCK_CASES)
+def test_moe_several_row_blocks(case):
+    """The walk over row blocks: the next block's rows and words taken up during
+    the last superstep, x copies that wrap to its first chunk, stores between
+    counted waits; dead rows and odd block counts (d8: 3 and 1) across it."""
+    E, H, I, d, K, k, T, shared, dead = case
+    blocks = -(-max(H, I) // 256)
+    assert E * -(-blocks // 2) >= 512               # the grid rule's first step
+    print(f"moe row blocks {case}", flush=True)
+    rng = np.random.default_rng(sum(case[:7]))
+    blk, ms, sh, vec = _block(rng, E, H, I, d, K, k, shared, dead)
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).cuda().bfloat16()
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[:, 3] += 2.0                              # expert 3 gets a tile of many rows
+    assert moe_path(blk, T) == PATH_GROUPED
+    y = blk(x, torch.from_numpy(logits).cuda())
+    assert torch.equal(y, blk(x, torch.from_numpy(logits).cuda()))
+    kw = {}
+    if shared:
+        kw = dict(shared_gate=_spec(sh["gate"]), shared_up=_spec(sh["up"]), shared_down=_spec(sh["down"]),
+                  shared_gate_vec=vec)
+    assert_close(y.float().cpu().numpy(), _oracle(x, logits, ms, k, kw), what=f"moe row blocks {case}")
+
+
 def _oracle(x, logits, ms, k, kw):
     """vo.moe_layer of the routed experts plus the shared expert's term."""
     xf = x.float().cpu().numpy()
