@@ -283,7 +283,6 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
 #pragma unroll
     for (int c = 0; c < NBUF - 1; ++c) copy_next(c);
     load_w(rw, 0, w, sc);
-    drop_scales(0, sc);
     clear();
     wait_vmem();                                // the tables and the first chunks
     __syncthreads();
@@ -301,6 +300,7 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
                 if constexpr (C == 0) {
                     load_w(rn, last ? 0 : sb + 1, wn, sn);
                     asm volatile("" ::: "memory");
+                    if (last) drop_scales(sb, sc);
                 }
                 compute(cc, buf, w, sc);
                 // the next chunk's copies are in: of this wave's loads at most the
@@ -324,7 +324,6 @@ __device__ __forceinline__ void wide_body(const WideParams &p, int expert, int r
 #pragma unroll
                 for (int g = 0; g < GPB; ++g) sc[m][g] = sn[m][g];
             }
-            drop_scales(last ? 0 : sb + 1, sc);
         }
         store(rw);
         clear();
