@@ -137,7 +137,8 @@ __global__ void __launch_bounds__(256) k_embed_gather(const EmbedArgs a) {
 // chunks: a lane's eight outputs are one or two entries under one scale. The
 // general kernel divides 64-bit indexes by d and the group for every output
 // and reads code and scale again for each; 2048 rows of 4096, d4 K4096 (20 MB):
-// the kernel 25 us -> 9.3, the call 22.5 -> 14.7 (MI355X), which is its host path.
+// the kernel 24 us -> 8.9 (kernel trace, which adds a microsecond or two), call
+// to call 22.5 -> 15 (MI355X), of which the host path is the longer part now.
 template <int D>
 __global__ void __launch_bounds__(256) k_embed_blocks(const EmbedArgs a) {
     constexpr int NC = 8 / D;
@@ -281,7 +282,7 @@ int vqk_embed_gather(const vqk_weights *w, const void *ids, int32_t id_type, int
     const int64_t total = n * a.lanes_per_row;
     const int64_t blocks = (total + 255) / 256;
     // 32-bit indexes, 16-byte entries of d = 8 and 8-byte ones of d = 4: ahead of
-    // the general kernel wherever it applies (25 against 9.3 us, above)
+    // the general kernel wherever it applies (24 against 8.9 us, above)
     if (a.layout == kEmbBlocks && (a.D == 4 || a.D == 8) && a.G % 8 == 0 && a.vec_ok &&
         (reinterpret_cast<uintptr_t>(w->codebook) & 15) == 0 && total <= INT32_MAX && a.IN <= INT32_MAX) {
         if (a.D == 4) hipLaunchKernelGGL(k_embed_blocks<4>, dim3(unsigned(blocks)), dim3(256), 0, hipStream_t(stream), a);

@@ -8,15 +8,18 @@
 // 0..3 or 4..7, 128 KB -- and computes the half of the sum over those columns
 // of each code; the half sums (fp32) are added by the kernel that reads them.
 // Every lookup is then an 8-byte LDS read. The codes are read by both halves,
-// at about the same time on one XCD (neighbours in its dispatch order), so
-// mostly once from HBM (927 MB fetched for the gate and up projections below,
-// of 1.07 GB stored). x comes split the same way ([2][rows, IN / 2]).
+// on one XCD (neighbours in its dispatch order) and while their tiles are few
+// at about the same time: 0.69 GB fetched for gate and up of 64 tokens below,
+// of 0.61 GB live; 1.93 GB for 509 tokens, of 1.07 GB. x comes split the same
+// way ([2][rows, IN / 2]).
 // 509 tokens x 10 of 512 experts of 4096 x 1024 and a shared expert, d8 K16384
-// (MI355X): gate + up 690 us, down 302 us, the layer 2190 -> 980 us; 64 tokens,
-// a fifth of the rows dead, 848 -> 591 us. What bounds it now, by timing probes
-// of gate + up: 365 us without weight loads and lookups (products, scales,
-// barriers), 520 without the loads, 740 without the lookups: the words arrive
-// later than one superstep, and 128 registers a wave leave no room for two.
+// (MI355X, kernel trace, beside the shared expert): gate + up 631 us, down 267
+// us; the layer, call to call, 2190 -> 976 us; 64 tokens, a fifth of the rows
+// dead, 848 -> 590 us. What bounds it now, by timing probes of gate + up in one
+// session on a slower box (690 us whole there): 520 without the weight loads,
+// 365 without loads and lookups; leaving out the lookups or the x copies alone
+// gained nothing (740, 735). The words arrive later than one superstep, and 128
+// registers a wave leave no room for two.
 //
 // Workgroup = 16 waves x 32 weight rows; it keeps its table over several
 // tiles. A superstep is two 32-code blocks, one to each lane group of

@@ -9,11 +9,12 @@
 // lane group l / 32, which holds every other 32-code block of the row), and
 // each 1 KB x operand read from LDS feeds a 32 x 32 tile -- two of them where
 // gate and up run together. 2048 tokens x 8 of 256 experts of 2048 x 512, d4
-// K4096 (MI355X): gate + up 130 us (69 GFLOP), down 89 us (34 GFLOP), against
-// 3 x ~200 us. Of the 130, timing probes put ~86 us into everything but the
-// lookups and products (the 218 MB of weights, x copies, stores, start-up) and
-// ~65 us into those, half of it overlapped: two waves per SIMD (the sums of
-// 96 rows take the registers of four) leave latencies uncovered.
+// K4096 (MI355X, kernel trace): gate + up 135 us (69 GFLOP), down 92 us (34
+// GFLOP), against 3 x ~200 us. Timing probes (of 130 us in their session) put
+// ~86 us into everything but the lookups and products (the 218 MB of weights,
+// x copies, stores, start-up) and ~65 us into those, half of it overlapped: two
+// waves per SIMD (the sums of 96 rows take the registers of four) leave
+// latencies uncovered.
 //
 // Workgroup = 8 waves x 32 weight rows over one tile of rows. The weights'
 // words are loaded one superstep (2 blocks) ahead into registers. x is fp16
