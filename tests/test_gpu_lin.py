@@ -92,6 +92,26 @@ def test_linear_rows(d, K, packed, OUT, IN, dt):
         assert (np.abs(y - ref) <= bar).all(), (N, np.abs(y - ref).max(), bar.min())
 
 
+@pytest.mark.parametrize("d,bits", [(2, b) for b in range(8, 13)] +
+                         [(d, b) for d in (4, 8) for b in (8, 9, 10, 11, 12, 13, 14, 16)])
+def test_linear_rows_every_width(d, bits):
+    """Every code width: whole supersteps and a ragged one, x in place and (past
+    2^28 products) in operand order, the scale in fp32 and the decoded weight."""
+    rng = np.random.default_rng(10 * d + bits)
+    for OUT, IN, rows in ((33, 128 * d * 9 + 64, (3, 17)), (13201, 4160, (20, 40))):
+        m = make_module(rng, 1, OUT, IN, d, 2 ** bits)
+        w, keep = _desc(m)
+        cols = np.arange(OUT) if OUT < 100 else rng.choice(OUT, 60, replace=False)
+        sub = dict(m, codes=m["codes"][:, cols], scales=m["scales"][:, cols], OUT=len(cols))
+        for N in rows:
+            print(f"linear width d{d} bits {bits} {IN}->{OUT} N{N}", flush=True)
+            x = torch.from_numpy(rng.standard_normal((N, IN)).astype(np.float32)).cuda().half()
+            for fused in (64, 0):
+                ref, bar = _ref(sub, x, rounded=True, decoded=fused == 0)
+                y = _apply(w, x, fused=fused)[:, cols]
+                assert (np.abs(y - ref) <= bar).all(), (N, fused, np.abs(y - ref).max())
+
+
 @pytest.mark.parametrize("d,K,packed,IN", [
     (2, 1024, True, 4160), (2, 256, False, 4096), (4, 4096, True, 4160), (4, 1024, True, 4096),
     (4, 65536, False, 4096), (8, 16384, True, 4160), (8, 4096, True, 4096), (8, 65536, False, 4160)])
