@@ -1,7 +1,9 @@
 // Matrix-core VQ linear for a few rows of x: y[n, o] = sum_i x[n, i] * W[o, i],
 // the decode step of a dense linear (_dense_fused, vq_switch.py:3339-3434) for
-// 2..64 rows, and for one row where the block-per-lane GEMV (vqk_gemv.h) has
-// no fast form (more than 64 blocks per weight row, or a ragged last block).
+// 2..64 rows of layers large enough for it (lin_beats_gemv, lin_beats_seg in
+// vqk_lin.hip), and for every row count where the block-per-lane GEMV
+// (vqk_gemv.h) has no fast form (more than 64 blocks per weight row, or a
+// ragged last block).
 //
 // What bounds it: the LDS lookups of the decode (one table read per code) and,
 // with many rows, the x operand, so each weight is decoded ONCE for up to 64
